@@ -748,6 +748,11 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     constexpr int L = X4 + Traits<TYPE>::kTail;   // plus (three main types) one 4-byte load
     constexpr int SLICE = X4 * 16 + 4 * Traits<TYPE>::kTail;   // bytes of a tile one thread brings in
     constexpr bool kExactDma = is_main_type(TYPE);   // a thread's loads are exactly its slice
+    // Q6_K super-blocks are 210 bytes: a tile of R rows starts on any even byte unless R times the
+    // row's block count is a multiple of 8.  Such tiles are brought in from the 16-byte boundary in
+    // front of them and sit up to 14 bytes further on in their stage (the 64 bytes a thread brings in
+    // for its 52.5 leave room).
+    constexpr bool kShiftedTiles = TYPE == JL_Q6_K && !DUAL && !FULL;
 
     const int tid = threadIdx.x;
     const int nthreads = LEAN ? THREADS : (int)blockDim.x;
@@ -833,8 +838,9 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         const int64_t offset = (int64_t)local * half_bytes;
         const int64_t remain = (int64_t)seg_rows * row_bytes - offset;
         // (the fixed-geometry form is launched over whole tiles only, and tracks no segment's rows)
-        const int bytes = LEAN || remain >= half_bytes ? half_bytes : (int)remain;
-        const uint8_t *base = wseg + offset;
+        const int shift = kShiftedTiles ? (int)offset & 15 : 0;
+        const int bytes = (LEAN || remain >= half_bytes ? half_bytes : (int)remain) + shift;
+        const uint8_t *base = wseg + (offset - shift);
         const uint8_t *base_up = DUAL ? w_up_first + offset : base;
         uint8_t *dst = ring + st * stage_bytes;
         const bool whole = exact && (FULL || bytes == half_bytes);  // uniform
@@ -857,7 +863,9 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
                 const int wave_off = k < X4 ? (k * nthreads + wave * JL_WAVE) * 16
                                             : X4 * nthreads * 16 + wave * JL_WAVE * 4;
                 const uint8_t *src = (DUAL && slot_up[k] ? base_up : base) + slot_off[k];
-                if (slot_off[k] + width > bytes) src = wseg;
+                // (a shifted tile's last 16 bytes may run past its end, not past the weight's, whose
+                // bytes are a multiple of 16)
+                if (kShiftedTiles ? slot_off[k] >= bytes : slot_off[k] + width > bytes) src = wseg;
                 if (k < X4)
                     __builtin_amdgcn_global_load_lds((gvoid *)src, (lvoid *)(dst + wave_off), 16, 0, 0);
                 else
@@ -1118,9 +1126,10 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         if (!in_wave && it > 0) finish(tile - grid, (it - 1) & 1);
 
         float v = 0.f;
+        const uint32_t tile_shift = kShiftedTiles ? (uint32_t)((int64_t)tile * half_bytes) & 15 : 0;   // (one weight)
         if (active) {
             if constexpr (PACKED) v = slice_dot_lds_packed<TYPE>(ring0 + (it % kStages) * stage_bytes, r_lds, s, row_bytes, px);
-            else v = slice_dot_lds<TYPE>(ring0 + (it % kStages) * stage_bytes, r_lds, s, row_bytes, x, sx);
+            else v = slice_dot_lds<TYPE>(ring0 + (it % kStages) * stage_bytes + tile_shift, r_lds, s, row_bytes, x, sx);
         }
         if (in_wave) {
             v = group_sum(v, Sp);
@@ -1452,12 +1461,15 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     const bool dual = w_up != nullptr;
     // bytes a thread brings in per tile
     const int slice = type == JL_Q8_0 ? 68 : type == JL_Q6_K ? 64 : is_side_type(type) ? 48 : 36;
-    // Rows of 16 448 .. 32 768 columns, plain and residual projections of the three main types: the
-    // weight seen as [2 rows x n / 2] (the kernel's HALVES form); a half row is whole blocks, a tile
-    // -- four half rows, two rows -- whole 16-byte pieces.
-    if (is_main_type(type) && !dual && !rms && !xq && !cells && nseg == 1 && n > 16384 && n <= 32768 &&
+    // Rows of 16 448 .. 32 768 columns, plain and residual projections of the three main types and
+    // Q6_K: the weight seen as [2 rows x n / 2] (the kernel's HALVES form); a half row is whole blocks, a
+    // tile -- four half rows, two rows -- whole 16-byte pieces, or (Q6_K) the weight as a whole is.
+    // (Q6_K 3584 x 18 944, the down projection of a Qwen2.5-7B-shaped model:
+    // 29.3 us on the one-wave-per-row kernel, 22.4 us here)
+    if ((is_main_type(type) || type == JL_Q6_K) && !dual && !rms && !xq && !cells && nseg == 1 && n > 16384 && n <= 32768 &&
         n % 128 == 0 && (n / 2) % jl_block_elems(type) == 0 && w[0]->rows % 2 == 0 && ((uintptr_t)x & 15) == 0 &&
-        ((uintptr_t)w[0]->blocks & 15) == 0 && ((int64_t)2 * row_bytes) % 16 == 0) {
+        ((uintptr_t)w[0]->blocks & 15) == 0 &&
+        (type == JL_Q6_K ? w[0]->rows * (int64_t)row_bytes : (int64_t)2 * row_bytes) % 16 == 0) {
         GemvParams h{};
         h.nseg = 1;
         h.w[0] = w[0]->blocks;
@@ -1475,6 +1487,7 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
         switch (type) {
             case JL_Q8_0: return launch_tiles_of<JL_Q8_0, false, false, false, kWideThreads, 256, false, true, false, true>(ctx, h, kWideThreads, lds);
             case JL_Q4_0: return launch_tiles_of<JL_Q4_0, false, false, false, kWideThreads, 256, false, true, false, true>(ctx, h, kWideThreads, lds);
+            case JL_Q6_K: return launch_tiles_of<JL_Q6_K, false, false, false, kWideThreads, 256, false, true, false, true>(ctx, h, kWideThreads, lds);
             default: return launch_tiles_of<JL_Q4_K, false, false, false, kWideThreads, 256, false, true, false, true>(ctx, h, kWideThreads, lds);
         }
     }
@@ -1494,7 +1507,7 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
         R = (wide ? kWideThreads : 256) / Sp;
         half_rows = dual ? R / 2 : R;
         if (half_rows < 1) fast = false;
-        else if (((int64_t)half_rows * row_bytes) % 16 != 0) fast = false;
+        else if (((int64_t)half_rows * row_bytes) % 16 != 0) fast = fast && type == JL_Q6_K && !dual;   // (shifted tiles)
     }
     for (int i = 0; fast && i < nseg; i++) {
         if (((uintptr_t)w[i]->blocks & 15) != 0) fast = false;

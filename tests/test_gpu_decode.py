@@ -887,3 +887,38 @@ def test_rows_of_more_than_16384_columns(ctx, t, d, n):
     assert rel_err(added - base, ref, mag + np.abs(base) * 1e-6) < 2e-5
     assert bits_equal(got, runs[1][0]) and bits_equal(added, runs[1][1])
     w.free()
+
+
+@pytest.mark.parametrize("d,n", [(3584, 18944), (8, 16896), (24, 32256), (256, 11008), (1000, 3328), (600, 4864),
+                                 (776, 2816), (12, 18944), (10, 16896)])
+def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n):
+    """Rows of an odd number of 210-byte super-blocks: the tile kernel's tiles of one, two or four such
+    rows -- or of four half rows, past 16384 columns -- begin 2 .. 14 bytes off the 16-byte pieces they
+    are brought in by (the last case's weight is no multiple of 16 bytes: the one-wave-per-row kernel).
+    2e-5 of the magnitude sum as for every other form of these sums; same bits twice; the outputs behind
+    the last row stay."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
+    say("q6_k odd tiles", d, n)
+    raw = synthetic.weight(O.Q6_K, d, n, seed=7700 + d)
+    x = synthetic.activations(n, seed=7701)
+    base = synthetic.activations(d, seed=7702)
+    ref = O.matmul(O.Q6_K, raw, x, d, n)
+    mag = magnitude(O.Q6_K, raw, x, d, n)
+    w = upload(ctx, O.Q6_K, raw, d, n)
+    dx = ctx.from_numpy(x)
+    runs = []
+    for _ in range(2):
+        out = ctx.float_array(d + 8, fill=POISON)
+        acc = ctx.from_numpy(base.copy())
+        proj = QuantizedProjections(ctx, TornadoWorkspace(wrapX=acc))
+        proj.floatMatvec(dx, out, w, n, d)
+        proj.residualMatvec(dx, w, n, d)
+        ctx.sync()
+        runs.append((out.get(), acc.get()))
+    got, added = runs[0]
+    assert np.all(got[d:] == POISON)
+    assert rel_err(got[:d], ref, mag) < 2e-5
+    assert rel_err(added, ref.astype(np.float64) + base, mag + np.abs(base) * 6e-8) < 2e-5
+    assert bits_equal(got, runs[1][0]) and bits_equal(added, runs[1][1])
+    w.free()
