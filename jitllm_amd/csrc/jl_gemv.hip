@@ -213,31 +213,38 @@ __device__ __forceinline__ void mix_bytes4(float &acc, uint32_t v, float x0, flo
     mix_high(acc, odd, x3);
 }
 
-// Dot of a quarter of a Q6_K super-block (ql[128] | qh[64] | 16 signed scales | fp16 d,
-// J/tensor/standard/Q6_KFloatTensor.java:66-122) with 64 activations.  Quarter (h, upper): the
-// 64 ql bytes and 32 qh bytes of half h; element l < 32 of the quarter is nibble `upper` of ql[l]
-// with bits 4 upper .. 4 upper + 1 of qh[l] on top, element 32 + l nibble `upper` of ql[32 + l]
-// with bits 4 upper + 2 .. + 3 of qh[l].  w = d * scale * (q - 32) with one scale per 16 elements;
-// sx are the sums of the activations facing each 16.
-__device__ __forceinline__ float slice_dot_q6_k(const uint32_t (&ql)[16], const uint32_t (&qh)[8], uint32_t scales,
-                                                uint32_t dbits, int upper, const float (&x)[64],
+// Dot of 64 weights of a Q6_K super-block (ql[128] | qh[64] | 16 signed scales | fp16 d,
+// J/tensor/standard/Q6_KFloatTensor.java:66-122) with the activations facing them.  w = d * scale *
+// (q - 32) with one scale per 16 elements; sx are the sums of the activations facing each 16.
+// A thread's 64 are not 64 consecutive columns (one nibble of 64 ql bytes: it would read twice the bytes
+// it uses) but both nibbles of the 32 ql bytes 64 h + 32 p ...: the low ones are columns 128 h + 32 p ...,
+// with bits 2 p .. 2 p + 1 of qh[32 h + l] on top, the high ones columns 128 h + 64 + 32 p ..., with bits
+// 4 + 2 p .. 5 + 2 p.  Shifted into place, nibble and top bits are each one mask away from a binary16
+// subnormal: q * 2^-24 from a low nibble, q * 2^-20 from a high one (10 bits: 16 q is at most 1008).
+// 19 operations per eight weights, 23 and twice the funnel shifts in the order of columns.  The unpacking
+// bounds these kernels, not the memory (weights from HBM, before -> after: vocabulary projection
+// 128256 x 4096 91.7 -> 78.4 us, 151936 x 3584 97.5 -> 89.3 us, down projection 3584 x 18944 23.6 -> 20.7 us).
+__device__ __forceinline__ float slice_dot_q6_k(const uint32_t (&ql)[8], const uint32_t (&qh)[8], uint32_t scales_low,
+                                                uint32_t scales_high, uint32_t dbits, int p, const float (&x)[64],
                                                 const float (&sx)[4]) {
-    const int shl = 4 * upper;
+    const int left = 4 - 2 * p, right = 4 + 2 * p;
     float a[4] = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
     for (int j = 0; j < 8; j++) {
-        const uint32_t h = qh[j] >> shl;
-        const uint32_t v0 = ((ql[j] >> shl) & 0x0F0F0F0Fu) | ((h & 0x03030303u) << 4);
-        const uint32_t v1 = ((ql[8 + j] >> shl) & 0x0F0F0F0Fu) | ((h & 0x0C0C0C0Cu) << 2);
-        mix_bytes4(a[j >> 2], v0, x[4 * j], x[4 * j + 1], x[4 * j + 2], x[4 * j + 3]);
-        mix_bytes4(a[2 + (j >> 2)], v1, x[32 + 4 * j], x[32 + 4 * j + 1], x[32 + 4 * j + 2], x[32 + 4 * j + 3]);
+        const uint32_t v = ql[j], t = v >> 8, h = qh[j] << left, g = qh[j] >> right;
+        const NibblePairs n{(v & 0x000F000Fu) | (h & 0x00300030u), (v & 0x00F000F0u) | (h & 0x03000300u),
+                            (t & 0x000F000Fu) | (g & 0x00300030u), (t & 0x00F000F0u) | (g & 0x03000300u)};
+#pragma unroll
+        for (int b = 0; b < 4; b++) mix_byte(n, b, x[4 * j + b], x[32 + 4 * j + b], a[j >> 2], a[2 + (j >> 2)]);
     }
     const float d = jl_half_bits_to_float(dbits) * kTwo24;
     float acc = 0.f;
 #pragma unroll
     for (int g = 0; g < 4; g++) {
-        const float sc = (float)(int)(int8_t)(scales >> (8 * g));
-        acc = fmaf(sc, fmaf(-32.f * kTwoM24, sx[g], a[g]), acc);
+        const float sc = (float)(int)(int8_t)((g < 2 ? scales_low : scales_high) >> (8 * (g & 1)));
+        // (powers of two: the high nibbles' products are 16 times as large)
+        acc = g < 2 ? fmaf(sc, fmaf(-32.f * kTwoM24, sx[g], a[g]), acc)
+                    : fmaf(sc * 0.0625f, fmaf(-512.f * kTwoM24, sx[g], a[g]), acc);
     }
     return acc * d;
 }
@@ -611,24 +618,23 @@ __device__ __forceinline__ float slice_dot_lds(uint32_t stage, int r, int s, int
     } else if constexpr (TYPE == JL_Q6_K) {
         // Super-blocks are 210 bytes apart, so every other one starts two bytes off a dword.  The
         // LDS serves such reads, but at a fraction of its rate (measured: 40 % of the kernel's
-        // time): the quarter is read as aligned dwords from two bytes before where that is needed
+        // time): the bytes are read as aligned dwords from two bytes before where that is needed
         // and each dword put together from its two neighbours with a funnel shift of 0 or 16 bits.
         const uint32_t sb = row + (s >> 2) * 210;
-        const int h = (s >> 1) & 1;
+        const int h = (s >> 1) & 1, p = s & 1;
         const uint32_t off = sb & 2u, shift = off * 8;
-        uint32_t wl[17], wh[9], ql[16], qh[8];
-        lds_read_17(sb - off + 64 * h, wl);
+        uint32_t wl[9], wh[9], ql[8], qh[8];
+        lds_read_9(sb - off + 64 * h + 32 * p, wl);
         lds_read_9(sb - off + 128 + 32 * h, wh);
-        uint2 sc2;
-        uint32_t d;
-        asm volatile("ds_read2_b32 %0, %2 offset0:0 offset1:1\n\tds_read_u16 %1, %3\n\ts_waitcnt lgkmcnt(0)"
-                     : "=&v"(sc2), "=&v"(d) : "v"(sb - off + 192 + 4 * (s & 3)), "v"(sb + 208) : "memory");
+        uint32_t scales_low, scales_high, d;
+        asm volatile("ds_read_u16 %0, %3\n\tds_read_u16 %1, %3 offset:4\n\tds_read_u16 %2, %4\n\ts_waitcnt lgkmcnt(0)"
+                     : "=&v"(scales_low), "=&v"(scales_high), "=&v"(d) : "v"(sb + 192 + 8 * h + 2 * p), "v"(sb + 208) : "memory");
 #pragma unroll
-        for (int i = 0; i < 16; i++) ql[i] = __builtin_amdgcn_alignbit(wl[i + 1], wl[i], shift);
-#pragma unroll
-        for (int i = 0; i < 8; i++) qh[i] = __builtin_amdgcn_alignbit(wh[i + 1], wh[i], shift);
-        const uint32_t scales = __builtin_amdgcn_alignbit(sc2.y, sc2.x, shift);
-        return slice_dot_q6_k(ql, qh, scales, d, s & 1, x, sx);
+        for (int i = 0; i < 8; i++) {
+            ql[i] = __builtin_amdgcn_alignbit(wl[i + 1], wl[i], shift);
+            qh[i] = __builtin_amdgcn_alignbit(wh[i + 1], wh[i], shift);
+        }
+        return slice_dot_q6_k(ql, qh, scales_low, scales_high, d, p, x, sx);
     } else if constexpr (TYPE == JL_Q8_0) {
         uint32_t w[17];
         lds_read_17(row + s * 68, w);
@@ -1021,16 +1027,20 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         // (threads with no slice never use theirs: the dot product below is skipped for them)
         if constexpr (HALVES) {
             if (active) {
-                const float4 *src = (const float4 *)(x_first + ((r & 1) * S + s) * 64);
+                const float4 *src = (const float4 *)(x_first + ((r & 1) * S + (TYPE == JL_Q6_K ? s & ~1 : s)) * 64);
 #pragma unroll
                 for (int k = 0; k < 16; k++) {
-                    const float4 v4 = src[k];
+                    // (Q6_K: half s & 1 of two slices, see slice_dot_q6_k)
+                    const float4 v4 = TYPE == JL_Q6_K ? src[(k & 8) * 2 + (s & 1) * 8 + (k & 7)] : src[k];
                     x[4 * k] = v4.x; x[4 * k + 1] = v4.y; x[4 * k + 2] = v4.z; x[4 * k + 3] = v4.w;
                 }
             }
         } else if (active) {
 #pragma unroll
-            for (int k = 0; k < 4; k++) lds_read_16f(xs0 + s * 272 + k * 64, &x[k * 16]);
+            for (int k = 0; k < 4; k++) {
+                if constexpr (TYPE == JL_Q6_K) lds_read_16f(xs0 + ((s & ~1) + (k >> 1)) * 272 + (s & 1) * 128 + (k & 1) * 64, &x[k * 16]);
+                else lds_read_16f(xs0 + s * 272 + k * 64, &x[k * 16]);
+            }
         }
         if constexpr (TYPE == JL_Q6_K) {
 #pragma unroll
