@@ -1425,6 +1425,11 @@ int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, boo
         }
         if (p.rms_w) return launch_tiles_of<TYPE, DUAL, true>(ctx, p, threads, lds);
     } else {
+        // (Q6_K rows of 2304 ... 4032 columns: 151936 x 3584 89.3 -> 85.7 us against the
+        // general instance)
+        if constexpr (TYPE == JL_Q6_K && !DUAL) {
+            if (fixed && !full && threads == 256 && p.Sp == 64) return launch_tiles_of<TYPE, false, false, false, 256, 64, false, true>(ctx, p, threads, lds);
+        }
         if (full && threads == 256) {
             if (p.Sp == 32) return launch_tiles_of<TYPE, DUAL, false, false, 256, 32>(ctx, p, threads, lds);
             if (p.Sp == 64) return launch_tiles_of<TYPE, DUAL, false, false, 256, 64>(ctx, p, threads, lds);
