@@ -889,6 +889,14 @@ def test_rows_of_more_than_16384_columns(ctx, t, d, n):
     w.free()
 
 
+@pytest.mark.parametrize("t,d,n", [(O.Q8_0, 12, 19200), (O.Q8_0, 12, 19328), (O.Q4_K, 12, 26624), (O.Q4_K, 12, 27136),
+                                   (O.Q4_0, 12, 26880), (O.Q4_0, 12, 27008)])
+def test_two_halves_vector_beside_the_tile_or_not(ctx, t, d, n):
+    """The longest activation vectors that are staged in LDS beside a tile of half rows, and the shortest that are
+    read from global memory instead: the same bounds on both sides."""
+    test_rows_of_more_than_16384_columns(ctx, t, d, n)
+
+
 @pytest.mark.parametrize("d,n", [(3584, 18944), (8, 16896), (24, 32256), (256, 11008), (1000, 3328), (600, 4864),
                                  (776, 2816), (12, 18944), (10, 16896)])
 def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n):
@@ -922,3 +930,10 @@ def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n):
     assert rel_err(added, ref.astype(np.float64) + base, mag + np.abs(base) * 6e-8) < 2e-5
     assert bits_equal(got, runs[1][0]) and bits_equal(added, runs[1][1])
     w.free()
+
+
+@pytest.mark.parametrize("d,n", [(12, 18944), (12, 19456), (12, 3584), (10, 3584), (4, 3840), (8, 2304)])
+def test_q6_k_vector_staging_and_partial_rows(ctx, d, n):
+    """Q6_K half rows whose vector fits beside a tile and not, and rows of 33 .. 63 slices in whole tiles (the
+    fixed-geometry instance) and not (the general one)."""
+    test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n)
