@@ -88,6 +88,9 @@ __device__ __host__ constexpr int row_bytes_of(int slices) {
            : TYPE == JL_Q4_1 ? slices * 40 : TYPE == JL_Q5_0 ? slices * 44 : TYPE == JL_IQ4_XS ? slices * 34 : slices * 36;
 }
 
+// sums a thread keeps of its activations
+template <int TYPE> constexpr int kSums = TYPE == JL_Q6_K ? 8 : 4;
+
 __device__ __forceinline__ float ubyte(uint32_t v, int k) { return (float)((v >> (8 * k)) & 0xFFu); }
 __device__ __forceinline__ float sbyte(uint32_t v, int k) { return (float)(int)(int8_t)(v >> (8 * k)); }
 
@@ -227,38 +230,40 @@ __device__ __forceinline__ void mix_bytes4(float &acc, uint32_t v, float x0, flo
 
 // Dot of 64 weights of a Q6_K super-block (ql[128] | qh[64] | 16 signed scales | fp16 d,
 // J/tensor/standard/Q6_KFloatTensor.java:66-122) with the activations facing them.  w = d * scale *
-// (q - 32) with one scale per 16 elements; sx are the sums of the activations facing each 16.
+// (q - 32) with one scale per 16 elements.
 // A thread's 64 are not 64 consecutive columns (one nibble of 64 ql bytes: it would read twice the bytes
 // it uses) but both nibbles of the 32 ql bytes 64 h + 32 p ...: the low ones are columns 128 h + 32 p ...,
 // with bits 2 p .. 2 p + 1 of qh[32 h + l] on top, the high ones columns 128 h + 64 + 32 p ..., with bits
 // 4 + 2 p .. 5 + 2 p.  Shifted into place, nibble and top bits are each one mask away from a binary16
 // subnormal: q * 2^-24 from a low nibble, q * 2^-20 from a high one (10 bits: 16 q is at most 1008).
-// 19 operations per eight weights, 23 and twice the funnel shifts in the order of columns.  The unpacking
-// bounds these kernels, not the memory (weights from HBM, before -> after: vocabulary projection
-// 128256 x 4096 91.7 -> 78.4 us, 151936 x 3584 97.5 -> 89.3 us, down projection 3584 x 18944 23.6 -> 20.7 us).
+// 19 operations per eight weights, 23 and twice the funnel shifts in the order of columns.
+// The 16 products of a scale are two chains of eight, each beginning with the eight's offset `off`
+// (-32 times the sum of its activations, in the products' unit): as many operations as one chain of 16
+// that the offset is taken off at the end, and sums that stay small.  Error against float64 over 2048
+// rows of 11008 columns 1.59e-7, one chain 2.12e-7, the one-wave-per-row kernel 1.61e-7; the four more
+// values a thread keeps cost up to 2 % (14336 x 3072 10.1 -> 10.3 us), 1024-row calls gain as much.
+// One group's chains end before the next one's begin: all sixteen at once take 126 registers for 111.
 __device__ __forceinline__ float slice_dot_q6_k(const uint32_t (&ql)[8], const uint32_t (&qh)[8], uint32_t scales_low,
                                                 uint32_t scales_high, uint32_t dbits, int p, const float (&x)[64],
-                                                const float (&sx)[4]) {
+                                                const float (&off)[8]) {
     const int left = 4 - 2 * p, right = 4 + 2 * p;
-    float a[4] = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-    for (int j = 0; j < 8; j++) {
-        const uint32_t v = ql[j], t = v >> 8, h = qh[j] << left, g = qh[j] >> right;
-        const NibblePairs n{(v & 0x000F000Fu) | (h & 0x00300030u), (v & 0x00F000F0u) | (h & 0x03000300u),
-                            (t & 0x000F000Fu) | (g & 0x00300030u), (t & 0x00F000F0u) | (g & 0x03000300u)};
-#pragma unroll
-        for (int b = 0; b < 4; b++) mix_byte(n, b, x[4 * j + b], x[32 + 4 * j + b], a[j >> 2], a[2 + (j >> 2)]);
-    }
-    const float d = jl_half_bits_to_float(dbits) * kTwo24;
     float acc = 0.f;
 #pragma unroll
-    for (int g = 0; g < 4; g++) {
-        const float sc = (float)(int)(int8_t)((g < 2 ? scales_low : scales_high) >> (8 * (g & 1)));
+    for (int g = 0; g < 2; g++) {   // the 16 columns of scales_low's and of scales_high's byte g
+        float a[2] = {off[2 * g], off[2 * g + 1]}, b[2] = {off[4 + 2 * g], off[5 + 2 * g]};
+#pragma unroll
+        for (int j = 4 * g; j < 4 * g + 4; j++) {
+            const uint32_t v = ql[j], t = v >> 8, h = qh[j] << left, u = qh[j] >> right;
+            const NibblePairs n{(v & 0x000F000Fu) | (h & 0x00300030u), (v & 0x00F000F0u) | (h & 0x03000300u),
+                                (t & 0x000F000Fu) | (u & 0x00300030u), (t & 0x00F000F0u) | (u & 0x03000300u)};
+#pragma unroll
+            for (int k = 0; k < 4; k++) mix_byte(n, k, x[4 * j + k], x[32 + 4 * j + k], a[(j >> 1) & 1], b[(j >> 1) & 1]);
+        }
+        acc = fmaf((float)(int)(int8_t)(scales_low >> (8 * g)), a[0] + a[1], acc);
         // (powers of two: the high nibbles' products are 16 times as large)
-        acc = g < 2 ? fmaf(sc, fmaf(-32.f * kTwoM24, sx[g], a[g]), acc)
-                    : fmaf(sc * 0.0625f, fmaf(-512.f * kTwoM24, sx[g], a[g]), acc);
+        acc = fmaf((float)(int)(int8_t)(scales_high >> (8 * g)) * 0.0625f, b[0] + b[1], acc);
     }
-    return acc * d;
+    return acc * (jl_half_bits_to_float(dbits) * kTwo24);
 }
 
 // Dot of one Q4_1 block pair (40 bytes: fp16 d, m | 16 nibble bytes, twice;
@@ -572,7 +577,7 @@ __device__ __forceinline__ void lds_read_q4k(uint32_t hdr, uint32_t qs, uint4 &h
 
 template <int TYPE>
 __device__ __forceinline__ float slice_dot_lds(uint32_t stage, int r, int s, int row_bytes,
-                                               const float (&x)[64], const float (&sx)[4]) {
+                                               const float (&x)[64], const float (&sx)[kSums<TYPE>]) {
     const uint32_t row = stage + (uint32_t)(r * row_bytes);
     if constexpr (TYPE == JL_IQ4_XS) {
         // the 8-byte header and the 32 nibble bytes of quarter s & 3 (super-blocks are 136 bytes
@@ -1018,7 +1023,8 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     __builtin_amdgcn_s_barrier();
 
     float x[64];
-    float sx[4] = {0.f, 0.f, 0.f, 0.f};   // sums of the slice's activations by 32 (4-bit types) or 16 (Q6_K)
+    // sums of the slice's activations by 32 (4- and 5-bit types), or by 8 times the offset (Q6_K, slice_dot_q6_k)
+    float sx[kSums<TYPE>] = {};
     PackedX px;
     if constexpr (PACKED) {
         // the slice's 64 bytes, two scales and two sums straight from global memory (a few KB that
@@ -1062,11 +1068,10 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         }
         if constexpr (TYPE == JL_Q6_K) {
 #pragma unroll
-            for (int k = 0; k < 16; k++) {
-                sx[0] += x[k];
-                sx[1] += x[16 + k];
-                sx[2] += x[32 + k];
-                sx[3] += x[48 + k];
+            for (int k = 0; k < 8; k++) {
+                const float *e = &x[8 * k];
+                sx[k] = ((e[0] + e[1]) + (e[2] + e[3])) + ((e[4] + e[5]) + (e[6] + e[7]));
+                sx[k] *= k < 4 ? -32.f * kTwoM24 : -512.f * kTwoM24;
             }
         } else if constexpr (TYPE != JL_Q8_0) {   // Q4_0, Q4_K, Q5_K: by 32
 #pragma unroll

@@ -937,3 +937,34 @@ def test_q6_k_vector_staging_and_partial_rows(ctx, d, n):
     """Q6_K half rows whose vector fits beside a tile and not, and rows of 33 .. 63 slices in whole tiles (the
     fixed-geometry instance) and not (the general one)."""
     test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n)
+
+
+@pytest.mark.parametrize("n", [2304, 4352, 11008, 18944])
+def test_q6_k_tile_kernel_no_further_off_than_one_wave_per_row(ctx, n):
+    """The same rows on the tile kernel and -- one row fewer, so that the weight is no multiple of 16 bytes -- on the
+    one-wave-per-row kernel, both against float64: the tile kernel's error (2-norm over the rows) is no larger.  Over
+    2048 rows each norm is known to 1 / sqrt(2 * 2048) = 1.6 %, their ratio to 2.2 %; 1.08 leaves 3.5 times that.  (One
+    chain of sixteen products per scale was 1.3 - 1.4 times as far off.)"""
+    import np_models as NP
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
+    say("q6_k error", n)
+    d, row_bytes = 2048, n // 256 * 210
+    raw = np.asarray(synthetic.weight(O.Q6_K, d, n, seed=7800)).reshape(-1)
+    assert raw.size == d * row_bytes and raw.size % 16 == 0 and (raw.size - row_bytes) % 16 != 0 and raw.size >= 2 << 20
+    x = synthetic.activations(n, seed=7801)
+    # (d * scale * q is exact in float32: 11 + 8 + 5 bits)
+    ref = np.concatenate([NP.DEQUANT[O.Q6_K](raw[i * row_bytes:(i + 256) * row_bytes]).reshape(256, n).astype(np.float64)
+                          @ x.astype(np.float64) for i in range(0, d, 256)])
+    proj = QuantizedProjections(ctx, TornadoWorkspace())
+    dx = ctx.from_numpy(x)
+    errors = []
+    for rows in (d, d - 1):
+        w = upload(ctx, O.Q6_K, raw[:rows * row_bytes], rows, n)
+        out = ctx.float_array(rows, fill=POISON)
+        proj.floatMatvec(dx, out, w, n, rows)
+        ctx.sync()
+        errors.append(np.linalg.norm(out.get()[:d - 1] - ref[:d - 1]) / np.linalg.norm(ref[:d - 1]))
+        w.free()
+    print(f"q6_k {n}: tile {errors[0]:.3e}, one wave per row {errors[1]:.3e}", flush=True)
+    assert errors[0] <= 1.08 * errors[1]
