@@ -890,21 +890,33 @@ def test_rows_of_more_than_16384_columns(ctx, t, d, n):
 
 
 @pytest.mark.parametrize("t,d,n", [(O.Q8_0, 12, 19200), (O.Q8_0, 12, 19328), (O.Q4_K, 12, 26624), (O.Q4_K, 12, 27136),
-                                   (O.Q4_0, 12, 26880), (O.Q4_0, 12, 27008)])
+                                   (O.Q4_0, 12, 26880), (O.Q4_0, 12, 27008), (O.Q8_0, 1030, 19200), (O.Q8_0, 1030, 19328),
+                                   (O.Q4_K, 1030, 26624), (O.Q4_K, 1030, 27136), (O.Q4_0, 1030, 26880), (O.Q4_0, 1030, 27008)])
 def test_two_halves_vector_beside_the_tile_or_not(ctx, t, d, n):
     """The longest activation vectors that are staged in LDS beside a tile of half rows, and the shortest that are
-    read from global memory instead: the same bounds on both sides."""
+    read from global memory instead: the same bounds on both sides.  1030 rows are 515 tiles, so that a chip of 256
+    compute units takes two and three in a workgroup -- the second overwrites the place where the vector lay."""
     test_rows_of_more_than_16384_columns(ctx, t, d, n)
 
 
-@pytest.mark.parametrize("d,n", [(3584, 18944), (8, 16896), (24, 32256), (256, 11008), (1000, 3328), (600, 4864),
-                                 (776, 2816), (12, 18944), (10, 16896)])
-def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n):
-    """Rows of an odd number of 210-byte super-blocks: the tile kernel's tiles of one, two or four such
-    rows -- or of four half rows, past 16384 columns -- begin 2 .. 14 bytes off the 16-byte pieces they
-    are brought in by (the last case's weight is no multiple of 16 bytes: the one-wave-per-row kernel).
-    2e-5 of the magnitude sum as for every other form of these sums; same bits twice; the outputs behind
-    the last row stay."""
+def q6_k_takes_the_tile_kernel(d, n):
+    """The row lengths, alignments and sizes of a plain Q6_K projection that the tile kernel serves (jl_launch_gemv)."""
+    row_bytes = n // 256 * 210
+    if 16384 < n <= 32768 and n % 512 == 0 and d % 2 == 0 and d * row_bytes % 16 == 0:
+        return True
+    return 2048 <= n <= 16384 and d * row_bytes % 16 == 0 and d * row_bytes >= 2 << 20
+
+
+@pytest.mark.parametrize("d,n,tile", [(3584, 18944, True), (8, 16896, True), (24, 32256, True), (256, 11008, True), (1000, 3328, True),
+                                      (600, 4864, True), (1000, 2816, True), (12, 18944, True), (600, 4608, True), (192, 15872, True),
+                                      (776, 2816, False), (10, 16896, False)])
+def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n, tile):
+    """Rows of an odd number of 210-byte super-blocks (or of twice that, or of 62): the tile kernel's tiles of one, two
+    or four such rows -- or of four half rows, past 16384 columns -- begin 2 .. 14 bytes off the 16-byte pieces they
+    are brought in by.  (The last two go to the one-wave-per-row kernel: less than 2 MB, and a weight that is no
+    multiple of 16 bytes.)  2e-5 of the magnitude sum as for every other form of these sums; same bits twice; the
+    outputs behind the last row stay."""
+    assert q6_k_takes_the_tile_kernel(d, n) == tile
     from jitllm_amd import synthetic
     from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
     say("q6_k odd tiles", d, n)
@@ -932,11 +944,49 @@ def test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n):
     w.free()
 
 
-@pytest.mark.parametrize("d,n", [(12, 18944), (12, 19456), (12, 3584), (10, 3584), (4, 3840), (8, 2304)])
+@pytest.mark.parametrize("d,n", [(12, 18944), (12, 19456), (1032, 18944), (1032, 19456), (1024, 3584), (1000, 3840), (1200, 2304),
+                                 (834, 3072), (1201, 4096)])
 def test_q6_k_vector_staging_and_partial_rows(ctx, d, n):
-    """Q6_K half rows whose vector fits beside a tile and not, and rows of 33 .. 63 slices in whole tiles (the
-    fixed-geometry instance) and not (the general one)."""
-    test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n)
+    """Q6_K half rows whose vector fits beside a tile and not, one tile a workgroup and several, and rows of 36 .. 60
+    slices in whole tiles that start on a 16-byte boundary (3584 columns) and off it: the fixed-geometry instance.  The
+    last two end in a ragged tile, the general instance (rows of 64 slices: 1201 is no multiple of four)."""
+    test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n, True)
+
+
+@pytest.mark.parametrize("d,n", [(1200, 2304), (1024, 3584), (256, 11008), (16, 18944)])
+def test_q6_k_values_that_are_not_finite(ctx, d, n):
+    """An infinite or NaN block scale reaches its own row and no other; an infinite or NaN activation reaches every row
+    (the 32 taken off every weight is taken off the activations' sum).  Finite rows keep their bits."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
+    say("q6_k not finite", d, n)
+    assert q6_k_takes_the_tile_kernel(d, n)
+    blocks = n // 256
+    raw = np.array(synthetic.weight(O.Q6_K, d, n, seed=7900)).reshape(d, blocks, 210)
+    x = synthetic.activations(n, seed=7901)
+    bad = {0: (0, np.inf), d // 2 + 1: (blocks - 1, np.nan), d - 1: (blocks // 2, -np.inf)}
+    spoilt = raw.copy()
+    for row, (block, value) in bad.items():
+        spoilt[row, block, 208:] = np.array([value], np.float16).view(np.uint8)
+    proj = QuantizedProjections(ctx, TornadoWorkspace())
+
+    def run(blocks_, x_):
+        w = upload(ctx, O.Q6_K, blocks_.reshape(-1), d, n)
+        out = ctx.float_array(d, fill=POISON)
+        proj.floatMatvec(ctx.from_numpy(x_), out, w, n, d)
+        ctx.sync()
+        got = out.get()
+        w.free()
+        return got
+
+    want, got = run(raw, x), run(spoilt, x)
+    rows = np.array(sorted(bad))
+    assert np.all(np.isfinite(want)) and not np.any(np.isfinite(got[rows]))
+    assert bits_equal(np.delete(got, rows), np.delete(want, rows))
+    for at, value in ((0, np.inf), (n - 1, np.nan), (n // 2 + 17, -np.inf)):
+        hit = x.copy()
+        hit[at] = value
+        assert not np.any(np.isfinite(run(raw, hit)))
 
 
 @pytest.mark.parametrize("n", [2304, 4352, 11008, 18944])
