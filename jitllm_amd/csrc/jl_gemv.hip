@@ -137,6 +137,12 @@ __device__ __forceinline__ void mix_low(float &acc, uint32_t w, float x) {
 __device__ __forceinline__ void mix_high(float &acc, uint32_t w, float x) {
     asm("v_fma_mix_f32 %0, %1, %2, %0 op_sel:[1,0,0] op_sel_hi:[1,0,0]" : "+v"(acc) : "v"(w), "v"(x));
 }
+// from + (binary16 in the low half of w) * x: the first product of a chain that begins with a value to be kept
+__device__ __forceinline__ float mix_low_from(float from, uint32_t w, float x) {
+    float acc;
+    asm("v_fma_mix_f32 %0, %1, %2, %3 op_sel:[0,0,0] op_sel_hi:[1,0,0]" : "=v"(acc) : "v"(w), "v"(x), "v"(from));
+    return acc;
+}
 // byte b (0..3) of the dword the pairs came from: acc_lo += low nibble * 2^-24 * x_lo,
 // acc_hi += high nibble * 2^-20 * x_hi
 __device__ __forceinline__ void mix_byte(const NibblePairs &n, int b, float x_lo, float x_hi, float &acc_lo,
@@ -241,9 +247,9 @@ __device__ __forceinline__ void mix_bytes4(float &acc, uint32_t v, float x0, flo
 // The 16 products of a scale are two chains of eight, each beginning with the eight's offset `off`
 // (-32 times the sum of its activations, in the products' unit): as many operations as one chain of 16
 // that the offset is taken off at the end, and sums that stay small.  Error against float64 over 2048
-// rows of 11008 columns 1.59e-7, one chain 2.12e-7, the one-wave-per-row kernel 1.61e-7; the four more
-// values a thread keeps cost up to 2 % (14336 x 3072 10.1 -> 10.3 us), 1024-row calls gain as much.
-// One group's chains end before the next one's begin: all sixteen at once take 126 registers for 111.
+// rows of 11008 columns 1.59e-7, one chain 2.12e-7, the one-wave-per-row kernel 1.61e-7; 4096 x 11008
+// 12.4 us, with one chain 12.6, and over 200 shapes 0.99 of the time.  One group's chains end before the
+// next one's begin: all sixteen at once take 126 registers for 111.
 __device__ __forceinline__ float slice_dot_q6_k(const uint32_t (&ql)[8], const uint32_t (&qh)[8], uint32_t scales_low,
                                                 uint32_t scales_high, uint32_t dbits, int p, const float (&x)[64],
                                                 const float (&off)[8]) {
@@ -251,14 +257,22 @@ __device__ __forceinline__ float slice_dot_q6_k(const uint32_t (&ql)[8], const u
     float acc = 0.f;
 #pragma unroll
     for (int g = 0; g < 2; g++) {   // the 16 columns of scales_low's and of scales_high's byte g
-        float a[2] = {off[2 * g], off[2 * g + 1]}, b[2] = {off[4 + 2 * g], off[5 + 2 * g]};
+        float a[2], b[2];
 #pragma unroll
         for (int j = 4 * g; j < 4 * g + 4; j++) {
             const uint32_t v = ql[j], t = v >> 8, h = qh[j] << left, u = qh[j] >> right;
             const NibblePairs n{(v & 0x000F000Fu) | (h & 0x00300030u), (v & 0x00F000F0u) | (h & 0x03000300u),
                                 (t & 0x000F000Fu) | (u & 0x00300030u), (t & 0x00F000F0u) | (u & 0x03000300u)};
+            const int c = (j >> 1) & 1;
 #pragma unroll
-            for (int k = 0; k < 4; k++) mix_byte(n, k, x[4 * j + k], x[32 + 4 * j + k], a[(j >> 1) & 1], b[(j >> 1) & 1]);
+            for (int k = 0; k < 4; k++) {
+                if (k == 0 && (j & 1) == 0) {
+                    a[c] = mix_low_from(off[j >> 1], n.lo02, x[4 * j]);
+                    b[c] = mix_low_from(off[4 + (j >> 1)], n.hi02, x[32 + 4 * j]);
+                } else {
+                    mix_byte(n, k, x[4 * j + k], x[32 + 4 * j + k], a[c], b[c]);
+                }
+            }
         }
         acc = fmaf((float)(int)(int8_t)(scales_low >> (8 * g)), a[0] + a[1], acc);
         // (powers of two: the high nibbles' products are 16 times as large)
@@ -364,7 +378,7 @@ __device__ __forceinline__ float slice_dot_q5_k(const uint4 &h, const uint32_t (
     }
     // (the scales behind the products: left to the compiler they go in front, where launches of one or two tiles a
     // workgroup lose up to 4 % against scales taken one by one, a branch each -- 4096 x 2048: one by one 3.78 us, in
-    // front 3.93, behind 3.83; 14336 x 8192: 20.3, 21.0, 19.9; 8192 x 16384: 38.2, 35.2, 35.2)
+    // front 3.93, behind 3.83; 14336 x 8192: 20.3, 21.0, 20.2; 8192 x 16384: 38.3, 35.2, 35.3)
     __builtin_amdgcn_sched_barrier(0);
     const uint32_t sm = k_scales(h.y, h.z, h.w, pair);
     float lo_term = ((d * ubyte(sm, 0)) * kTwo24) * (a0 + a1) - (dmin * ubyte(sm, 2)) * sx[0];
