@@ -8,7 +8,8 @@ launches, 1 316 320 256 algorithmic bytes (weights in GGUF block layout + fp32 i
 each once).  Inputs are resident in HBM before the timed region.  Every layer owns distinct device
 buffers, so the 1.3 GB sweep cannot live in the 256 MB memory-side cache.
 
-Prints one JSON line.  `value` is GB/s of algorithmic bytes; `roofline` is the largest single
+Prints one JSON line of at most RESULT_LINE_LIMIT characters, and to stderr the full record behind it
+(every leg's statistics, checks and descriptions) as another.  `value` is GB/s of algorithmic bytes; `roofline` is the largest single
 launch shape of the step (the fused gate/up GEMV) against the 8 TB/s HBM peak; `cpu_baseline` is the
 oracle's restatement of the reference's Java CPU matmul timed on this machine's host cores;
 `prefill` and `batched` carry the MFMA side of the metric.
@@ -1135,6 +1136,34 @@ def int8_probe(ctx, t, T=2048):
                                             "gate/up": T * 2 * HIDDEN * DIM, "down": T * HIDDEN * DIM}}))
 
 
+# What a leg's record holds beside its results: in the full record, not in the result line.
+LEG_DETAIL = {"ms_stats", "us_stats", "launch_us_stats", "cpu_baseline", "check_rel_err", "math", "weights_from", "sustained_from_box",
+              "peak_from_box", "kernel", "layer", "weight", "what", "note", "sample", "layers_swept", "copies_swept", "bytes",
+              "weight_bytes", "bytes_per_layer", "bytes_per_launch", "flops_per_launch", "peak", "unit", "bound", "flop_per_byte",
+              "shapes", "host", "tok_s_per_layer", "rms_apply_to_fp16_us"}
+RESULT_LINE_LIMIT = 8000
+
+
+def result_line(out) -> str:
+    """The one line of JSON a run prints: every plain value, the workload, the checks and the roofline as they are, of the
+    other legs the results.  A reader may keep only so many characters of a line, so it stays below RESULT_LINE_LIMIT: legs
+    that do not fit are named in "legs_in_full_record_only" (the last ones first)."""
+    def results(v, leg):
+        if isinstance(v, dict):
+            # (shares of a peak: of the two legs that the metric is about; elsewhere the rate says the same)
+            return {k: results(x, leg) for k, x in v.items()
+                    if k not in LEG_DETAIL and (leg in ("prefill", "decode_kernels") or not k.startswith("frac_"))}
+        return [results(x, leg) for x in v] if isinstance(v, list) else v
+
+    whole = ("config", "checks_rel_err", "ms_per_step_stats", "roofline", "cpu_baseline")
+    legs = [k for k, v in out.items() if isinstance(v, (dict, list)) and k not in whole]
+    line = {k: results(v, k) if k in legs else v for k, v in out.items()}
+    while len(json.dumps(line)) > RESULT_LINE_LIMIT and legs:
+        line.setdefault("legs_in_full_record_only", []).append(legs[-1])
+        del line[legs.pop()]
+    return json.dumps(line)
+
+
 def main():
     ap = argparse.ArgumentParser()
     ap.add_argument("--gpus", type=int, default=1)
@@ -1424,7 +1453,8 @@ def main():
             # between batched decode and prefill: 96, 192 and 384 rows (most prompts are this long)
             out["short_prompt"] = bench_short_prompt(ctx, hip, (96, 192, 384), max(5, args.steps // 5), 3)
         out["cpu_baseline"] = cpu_baseline(host, shapes, t) if cpu else None
-    print(json.dumps(out))
+    print(json.dumps({"full_record": out}), file=sys.stderr, flush=True)
+    print(result_line(out), flush=True)
 
 
 if __name__ == "__main__":

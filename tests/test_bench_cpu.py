@@ -34,3 +34,21 @@ def test_more_than_one_gpu_is_refused_in_words():
     assert proc.returncode != 0
     assert "one GPU" in (proc.stdout + proc.stderr)
     assert not proc.stdout.strip().startswith("{")
+
+
+def test_the_result_line_stays_short():
+    """Statistics and prose of the legs stay out of the printed line, and so do whole legs where that is not enough; the
+    plain values, the workload and the roofline are always in it."""
+    import json
+    import bench
+    out = {"metric": "m", "value": 1.5, "steps": 3, "config": {"workload": "w"}, "roofline": {"bound": "hbm", "frac": 0.5},
+           "prefill": [{"tokens": 512, "ms_per_layer": 0.1, "ms_stats": {"median": 0.1}, "roofline": {"kernel": "k", "frac": 0.4}}],
+           "big": [{"B": b, "note": "x" * 500, "GB_s": b + 0.5} for b in range(40)],
+           "short_prompt": [{"tokens": t} for t in range(3000)], "cpu_baseline": None}
+    text = bench.result_line(out)
+    line = json.loads(text)
+    assert "\n" not in text and len(text) <= bench.RESULT_LINE_LIMIT
+    assert all(line[k] == out[k] for k in ("metric", "value", "steps", "config", "roofline", "cpu_baseline"))
+    assert line["prefill"] == [{"tokens": 512, "ms_per_layer": 0.1, "roofline": {"frac": 0.4}}]
+    assert line["big"][3] == {"B": 3, "GB_s": 3.5} and line["legs_in_full_record_only"] == ["short_prompt"]
+    assert len(out["big"][0]["note"]) == 500
