@@ -190,8 +190,9 @@ __device__ __forceinline__ float slice_dot_q4_0(const uint32_t (&dw)[9], const f
 // the 12 packed bytes of a super-block (a | b | c: low four of the scales and of the minimums with two
 // spare bits each on top, then the nibbles of the high four).  A thread's pair is the same for the whole kernel, so
 // the selector and the masks are set up once and four values cost seven operations and a conversion each, where
-// each taken on its own cost about eight.  (The kernels are bound by their vector instructions: 2 x [18944 x 3584] gate/up with
-// RMS folding 21.1 -> 20.1 us, 3584 x 18944 13.8 -> 13.3 us, weights from HBM.)
+// each taken on its own cost about eight.  (Two thirds of the gate/up launches' time is the issue of their vector
+// instructions: Q4_K 2 x [18944 x 3584] with RMS folding 8.49 -> 8.03 million of them, 13.1 of its 20.3 us; plain
+// projections of Q4_K 0.95 - 1.00 of the time with values taken one by one.)
 __device__ __forceinline__ uint32_t k_scales(uint32_t a, uint32_t b, uint32_t c, int pair) {
     const uint32_t sel = pair & 1 ? 0x07060302u : 0x05040100u;
     const uint32_t own = pair < 2 ? 0x3F3F3F3Fu : 0x0F0F0F0Fu, top = pair < 2 ? 0u : 0x30303030u;
@@ -765,7 +766,8 @@ __device__ __forceinline__ uintptr_t uniform_value(uintptr_t v) {
 // vector, odd rows the second.  A tile holds four such half rows, so a thread always serves the same
 // half and keeps its 64 activations in registers as ever; they are staged through LDS where the vector
 // and the first tile fit there together (read lane by lane, 256 bytes apart, every load touches 64 cache lines:
-// 3584 x 18944 Q4_K 16.8 -> 13.8 us, Q6_K 20.7 -> 18.0 us, staged), and else come straight from global memory.  The thread that finishes a row adds its two halves'
+// Q4_K 3584 x 18944 16.8 us so, 13.8 staged), and else come straight from global memory.  The vector's place is
+// rounded up to whole passes of the workgroup, 16 KB.  The thread that finishes a row adds its two halves'
 // partial sums.)
 template <int TYPE, bool DUAL, bool RMS, bool PACKED = false, int THREADS = 256, int SPT = 0, bool SEGS = false,
           bool PART = false, bool ARGMAX = false, bool HALVES = false>
@@ -1042,7 +1044,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     __builtin_amdgcn_s_barrier();
 
     float x[64];
-    // sums of the slice's activations by 32 (4- and 5-bit types), or by 8 times the offset (Q6_K, slice_dot_q6_k)
+    // sums of the slice's activations by 32 (4- and 5-bit types); Q6_K: the offsets of its chains of 8 (slice_dot_q6_k)
     float sx[kSums<TYPE>] = {};
     PackedX px;
     if constexpr (PACKED) {
@@ -1426,7 +1428,8 @@ int launch_fixed(jl_context *ctx, const GemvParams &p, int lds, bool full) {
 // weight).  The three main types have an instance for every variant at row lengths of 513 ... 8192
 // columns and, in the 1024-thread form (plain and residual), up to 16384 -- and, a row taken as two
 // half rows, up to 32768 (launched from jl_launch_gemv itself); the side types for whole rows of
-// 2048, 4096 and (plain and residual) 8192 columns.
+// 2048, 4096 and (plain and residual) 8192 columns, Q6_K also for plain and residual rows of 2304 ... 3840
+// columns and, as two half rows, of 16896 ... 32768.
 template <int TYPE, bool DUAL>
 int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed, int *cells = nullptr) {
     // (side types: plain, residual and gate/up only -- the caller has refused the rest)
@@ -1468,8 +1471,8 @@ int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, boo
         }
         if (p.rms_w) return launch_tiles_of<TYPE, DUAL, true>(ctx, p, threads, lds);
     } else {
-        // (Q6_K rows of 2304 ... 4032 columns: 151936 x 3584 89.3 -> 85.7 us against the
-        // general instance)
+        // (Q6_K rows of 2304 ... 3840 columns, 36 ... 60 of 64 slices: 151936 x 3584 89.3 us on the general instance,
+        // 85.7 on this one.  Rows of 65 ... 127 slices have none: not tried)
         if constexpr (TYPE == JL_Q6_K && !DUAL) {
             if (fixed && !full && threads == 256 && p.Sp == 64) return launch_tiles_of<TYPE, false, false, false, 256, 64, false, true>(ctx, p, threads, lds);
         }
@@ -1532,8 +1535,9 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     // Rows of 16 448 .. 32 768 columns, plain and residual projections of the three main types and
     // Q6_K: the weight seen as [2 rows x n / 2] (the kernel's HALVES form); a half row is whole blocks, a
     // tile -- four half rows, two rows -- whole 16-byte pieces, or (Q6_K) the weight as a whole is.
-    // (Q6_K 3584 x 18 944, the down projection of a Qwen2.5-7B-shaped model:
-    // 29.3 us on the one-wave-per-row kernel, 22.4 us here)
+    // (Q6_K against the one-wave-per-row kernel, no size left out: 8 x 16 896 7.7 and 5.2 us, 3584 x 18 944, the down
+    // projection of a Qwen2.5-7B-shaped model, 30.0 and 18.5; where the vector is not staged 1024 x 19 456 11.5 and
+    // 11.5, 8192 x 31 744 92.7 and 45.5)
     if ((is_main_type(type) || type == JL_Q6_K) && !dual && !rms && !xq && !cells && nseg == 1 && n > 16384 && n <= 32768 &&
         n % 128 == 0 && (n / 2) % jl_block_elems(type) == 0 && w[0]->rows % 2 == 0 && ((uintptr_t)x & 15) == 0 &&
         ((uintptr_t)w[0]->blocks & 15) == 0 &&
@@ -1604,7 +1608,11 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     if (is_side_type(type)) {
         // measured: the tile kernel is the faster one from rows of 2048 columns and 2 MB of weights
         // (by up to 1.7 x on the vocabulary and feed-forward projections); below that the two are
-        // within a few tenths of a microsecond of each other and the one-wave-per-row kernel stays
+        // within a few tenths of a microsecond of each other and the one-wave-per-row kernel stays.
+        // (Q6_K rows whose tiles start off a 16-byte boundary, every super-block count from 9 to 63 at 2 MB, 1024,
+        // 3584, 8192 and 32768 rows: 0.44 - 0.94 of the one-wave-per-row kernel's time, also where half of a tile's
+        // threads have no slice -- 17 super-blocks: 592 rows 5.05 and 4.55 us, 8192 rows 16.8 and 12.1 -- and from 61,
+        // whose 256 threads take one row a tile: 168 rows 9.5 and 5.3, 8192 rows 48.9 and 38.5)
         if (!fast || n < 2048 || w[0]->bytes * (dual ? 2 : 1) < ((int64_t)2 << 20))
             return jl_launch_gemv_direct(ctx, w[0], w_up, x, outs[0], epilogue);
     }
