@@ -953,6 +953,28 @@ def test_q6_k_vector_staging_and_partial_rows(ctx, d, n):
     test_q6_k_tiles_that_start_off_a_16_byte_boundary(ctx, d, n, True)
 
 
+@pytest.mark.parametrize("d,n", [(836, 3072)])
+def test_q6_k_fixed_geometry_and_general_instances_give_the_same_bits(ctx, d, n):
+    """Rows of 48 of 64 slices: whole tiles of four rows run the fixed-geometry instance, two rows more the general one;
+    the rows they share have the same bits.  (Lengths whose tiles start off a 16-byte boundary, 2304 and 3840
+    columns, allow no ragged tile, and 3584 none either; rows of 32 or 64 whole slices have the block's scale contracted
+    into the first sum of two lanes, where the general instance rounds the product.)"""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
+    say("q6_k fixed vs general", d, n)
+    raw = np.asarray(synthetic.weight(O.Q6_K, d + 2, n, seed=7950)).reshape(d + 2, -1)
+    dx = ctx.from_numpy(synthetic.activations(n, seed=7951))
+    proj = QuantizedProjections(ctx, TornadoWorkspace())
+    got = []
+    for rows in (d, d + 2):
+        assert q6_k_takes_the_tile_kernel(rows, n) and rows % 4 == (rows - d)
+        out = ctx.float_array(rows, fill=POISON)
+        proj.floatMatvec(dx, out, upload(ctx, O.Q6_K, raw[:rows].reshape(-1), rows, n), n, rows)
+        ctx.sync()
+        got.append(out.get())
+    assert np.all(got[1] != POISON) and bits_equal(got[0], got[1][:d])
+
+
 @pytest.mark.parametrize("d,n", [(1200, 2304), (1024, 3584), (256, 11008), (16, 18944)])
 def test_q6_k_values_that_are_not_finite(ctx, d, n):
     """An infinite or NaN block scale reaches its own row and no other; an infinite or NaN activation reaches every row
