@@ -13,6 +13,10 @@
 //     rounded once to fp16, which is what the reference's dequantize*ToFP16 kernels store;
 //   * the contraction runs on v_mfma_f32_16x16x32_f16 with fp32 accumulators;
 //   * epilogues: store, residual add, SwiGLU of a gate/up pair; rows past active_rows untouched.
+//
+// jl_launch_gemm, at the end, is where a call is given to this kernel or to one of the others: the
+// weight-streaming one (jl_gemm_skinny_kernels.h), the one that decodes in registers (jl_gemm_reg.hip), or
+// the fp16 GEMM over weights decoded once (jl_gemm_dense.hip).
 #include <stdlib.h>
 
 #include "jl_device.h"
@@ -968,12 +972,25 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     const double copy_us = kept && rows >= 128 ? 24.0 + 0.45 * ((rows + 255) / 256) * millions
                            : dense_only       ? 30.0 + 2.8 * millions
                                               : 1e30;
+    // ... and the kernel that decodes in registers, priced by its own table, at 65 .. 511 rows.  With Q4_K it
+    // rounds a weight to fp16, as the ways that decode in the loop or once do and the weight-streaming kernel
+    // does not: of that type it takes calls from those only, after the streaming kernel has had its choice.
+    // A call over a kept copy gives the bits of one without from 512 rows on and below 128: it is not
+    // considered from 512 on, nor where a copy is kept and read, and Q6_K (whose calls read a kept copy at any
+    // row count) comes here from 128 on.
+    int reg_tiling = -1;
+    double reg_us = 1e30;
+    if (rows < 512 && rows >= (dense_only ? 128 : 65) && !(kept && (rows >= 128 || dense_only)) && workspace_bytes >= head)
+        reg_us = jl_gemm_reg_price(ctx, weights, count, rows, epilogue, &reg_tiling);
     if (rows < 512) {
         // batched decode of up to 64 rows, and calls of up to 511 where it is the cheapest: the
         // weight-streaming kernel reads X itself, fp32 or fp16
         bool taken = false;
+        double other_us = in_loop_us < copy_us ? in_loop_us : copy_us;
+        // (near equal prices the streaming kernel is the faster one, by up to 8 %, measured)
+        if (1.1 * reg_us < other_us && type != JL_Q4_K) other_us = 1.1 * reg_us;
         int st = jl_launch_gemm_skinny(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue,
-                                       planes, plane_bytes, in_loop_us < copy_us ? in_loop_us : copy_us, &taken);
+                                       planes, plane_bytes, other_us, &taken);
         if (st != JL_OK || taken) return st;
     }
 
@@ -982,10 +999,11 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     // narrow weight are a few dozen 128 x 128 tiles, and K cut into runs is what fills the chip)
     const int dense_from = dense_only ? 1 : kept && copy_us < in_loop_us ? 128 : 512;
     int dsplits = 1, bm = 256;
-    int bn = jl_dense_column_tile(rows, k, virt, epilogue, ctx->compute_units, &dsplits, &bm, dense_from, ctx->split_k);
+    double dense_us = 1e30;
+    int bn = jl_dense_column_tile(rows, k, virt, epilogue, ctx->compute_units, &dsplits, &bm, dense_from, ctx->split_k, &dense_us);
     if (bn != 0 && dsplits > 1 && in_workspace + jl_dense_plane_bytes(rows, virt, dsplits) > plane_bytes) {
         // no room for the partial sums of a cut K: the cheapest tiling that keeps K whole
-        bn = jl_dense_column_tile(rows, k, virt, epilogue, ctx->compute_units, &dsplits, &bm, dense_from, false);
+        bn = jl_dense_column_tile(rows, k, virt, epilogue, ctx->compute_units, &dsplits, &bm, dense_from, false, &dense_us);
     }
     if (dense_only && bn == 0) {
         bn = 128;
@@ -1002,6 +1020,19 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
         }
         return jl_fail(JL_ERR_WORKSPACE, "jl_gemm: a %s weight needs room for its fp16 copy (%zu bytes) in the workspace",
                        jl_type_name(type), copy_bytes);
+    }
+    // The decoded copy's way (Q6_K) in microseconds: the GEMM, a launch that decodes the weights at 4.0 TB/s
+    // and converts the activations at 2.9, and 1.5 us between launches, all measured.  Both prices are those
+    // of fp32 activations whatever came: a call's sums do not depend on which of the two forms its
+    // activations have.
+    const double decoded_us = dense_us + 3.5 + (dsplits > 1 ? 1.5 : 0.0) + (weight_bytes + 2.0 * virt * k) / 4.0e6 + 6.0 * rows * k / 2.9e6;
+    if (reg_tiling >= 0 && reg_us < (dense ? decoded_us : in_loop_us)) {
+        if (!X16) {
+            hipLaunchKernelGGL(jl_rows_to_f16, dim3(rows), dim3(256), 0, ctx->stream, X, A, row_scale, rows, k);
+            JL_HIP(hipGetLastError());
+        }
+        return jl_launch_gemm_reg(ctx, weights, count, X16 ? X16 : A, X16 ? nullptr : row_scale, C, c_f16, rows, ldo,
+                                  col_offset, epilogue, reg_tiling);
     }
     // what a kept copy looks like: gate / up interleaved by half tiles of this BN, or plain
     const int32_t layout = epilogue == JL_SWIGLU ? bn : 1;

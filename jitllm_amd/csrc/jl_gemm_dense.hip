@@ -614,7 +614,7 @@ int launch_decode(jl_context *ctx, const DecodeParams &d, int activation_rows) {
 // only; not with `may_cut_k` false), which costs the fold's launch and the partial sums' trip
 // through memory.
 int jl_dense_column_tile(int rows, int k, int out_cols_virtual, int epilogue, int compute_units, int *splits,
-                         int *row_tile, int min_rows, bool may_cut_k) {
+                         int *row_tile, int min_rows, bool may_cut_k, double *us) {
     *splits = 1;
     *row_tile = 256;
     if (rows < min_rows || k % 64 != 0) return 0;
@@ -647,6 +647,7 @@ int jl_dense_column_tile(int rows, int k, int out_cols_virtual, int epilogue, in
             }
         }
     }
+    if (us && best_bn != 0) *us = best / per_us;
     return best_bn;
 }
 

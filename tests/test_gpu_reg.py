@@ -1,0 +1,135 @@
+"""Batched projections on the kernel that decodes weights in registers (jl_gemm_reg.hip): every tiling of
+every type it takes, at row counts and widths on and off the edges of its tiles, against the oracle."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from gpu_util import magnitude, rel_err, say
+from oracle import pyoracle as O
+
+pytestmark = pytest.mark.gpu
+
+# operands rounded once to fp16 (2^-11 each, of the weight and of the activation) and fp32 sums
+F16_BOUND = 2e-3
+UNTOUCHED = np.float32(-12345.5)
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    from jitllm_amd.runtime import Context
+    with Context(0) as c:
+        yield c
+
+
+def columns(d):
+    """The output columns that are checked: all of a narrow weight; of a wide one both ends, where tiles
+    and ragged last groups are, and a stride through the rest that meets every place in a tile."""
+    if d <= 600:
+        return np.arange(d)
+    return np.unique(np.concatenate([np.arange(40), np.arange(d - 70, d), np.arange(0, d, 131)]))
+
+
+def rows_of(raw, d, cols):
+    return np.ascontiguousarray(raw.reshape(d, -1)[cols]).reshape(-1)
+
+
+# (type, columns, weight rows side by side, activation rows, active, gate/up, residual): the 8 x 8, 7 x 8,
+# 7 x 4 x 2, 4 x 4 x 2, 4 x 4, 4 x 2 x 2 and 2 x 2 x 2 tilings of Q4_0, then what the other types have of
+# them, as the kernel's price list chooses (a kernel trace of this file shows every instance); one block of columns (a set of waves idle), odd block counts, rows of one group, weights whose
+# last group overlaps the one before
+CASES = [
+    (O.Q4_0, 256, (14003, 14003), 449, 449, True, False), (O.Q4_0, 256, (10001, 10001), 257, 257, True, False),
+    (O.Q4_0, 512, (14003, 14003), 65, 65, True, False), (O.Q4_0, 512, (5005,), 300, 300, False, True),
+    (O.Q4_0, 256, (14003, 14003), 97, 97, True, False), (O.Q4_0, 512, (10001,), 129, 129, False, False),
+    (O.Q4_0, 256, (16,), 65, 65, False, True), (O.Q4_0, 256, (100, 17, 33), 65, 65, False, True),
+    (O.Q8_0, 256, (14003, 14003), 449, 449, True, False), (O.Q8_0, 256, (10001, 10001), 257, 257, True, False),
+    (O.Q8_0, 512, (12001,), 257, 257, False, True), (O.Q8_0, 256, (12001, 12001), 200, 199, True, False),
+    (O.Q8_0, 512, (3003, 3003), 257, 257, True, False), (O.Q8_0, 512, (3003, 17, 100), 65, 65, False, False),
+    (O.Q4_K, 512, (14003, 14003), 449, 449, True, False), (O.Q4_K, 2304, (16390, 16390), 65, 65, True, False),
+    (O.Q4_K, 2816, (8200, 8200), 97, 97, True, False), (O.Q4_K, 2816, (2050, 2050), 384, 384, True, False),
+    (O.Q4_K, 2304, (6007, 6007), 257, 257, True, False), (O.Q4_K, 2816, (1002, 1002), 449, 440, True, False),
+    (O.Q6_K, 5888, (5005,), 200, 200, False, True),
+    (O.Q6_K, 256, (33,), 128, 128, False, True), (O.Q6_K, 512, (4099,), 128, 128, False, False),
+    (O.Q6_K, 768, (4099, 4099), 128, 128, True, False), (O.Q6_K, 2816, (40, 17), 140, 130, False, False),
+    (O.Q6_K, 768, (100, 100), 160, 145, True, False),
+]
+
+
+@pytest.mark.parametrize("t,n,ds,rows,active,dual,residual", CASES)
+def test_weights_decoded_in_registers(ctx, t, n, ds, rows, active, dual, residual):
+    """Against the oracle for fp32 activations; binary16 ones of the same values give the same bits, a
+    second call gives the same bits as the first, rows past the active ones stay as they were."""
+    from jitllm_amd import _lib as L, synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("decode in registers", t, n, ds, rows, active, dual, residual)
+    raws = [synthetic.weight(t, d, n, seed=7100 + i) for i, d in enumerate(ds)]
+    ws = [ctx.load_weight(t, raw, d, n) for raw, d in zip(raws, ds)]
+    X = synthetic.activations((rows, n), seed=7110).astype(np.float16).astype(np.float32)
+    width = ds[0] if dual else sum(ds)
+    base = synthetic.activations((rows, width), seed=7111) if residual else np.full((rows, width), UNTOUCHED, np.float32)
+    proj = QuantizedBatchProjections(ctx, rows, n, sum(ds))
+    ep = L.JL_SWIGLU if dual else L.JL_RESIDUAL if residual else L.JL_STORE
+    outs = []
+    for x in (ctx.from_numpy(X), ctx.from_numpy(X), ctx.half_from_numpy(X.astype(np.float16))):
+        out = ctx.from_numpy(base.reshape(-1).copy())
+        proj._gemm(ws, x, out, active, width, 0, ep)
+        ctx.sync()
+        outs.append(out.get().reshape(rows, width))
+        out.free()
+        x.free()
+    for other in outs[1:]:
+        assert np.array_equal(outs[0].view(np.uint32), other.view(np.uint32))
+    got = outs[0]
+    assert np.array_equal(got[active:], base[active:])
+    if dual:
+        cols = columns(width)
+        parts = [rows_of(raw, width, cols) for raw in raws]
+        g, u = (O.matmul_batch(t, part, X[:active], len(cols), n) for part in parts)
+        mg, mu = (magnitude(t, part, X[:active], len(cols), n) for part in parts)
+        # an error of gate enters with SiLU's slope (at most 1.1) times up, one of up with SiLU(gate) <= |gate|
+        sig = 1.0 / (1.0 + np.exp(-g.astype(np.float64)))
+        bound = F16_BOUND * (1.1 * mg * np.abs(u) + np.abs(g) * sig * mu + 1.1 * F16_BOUND * mg * mu) + 1e-5
+        assert np.all(np.abs(got[:active, cols] - g * sig * u) <= bound)
+    else:
+        at = 0
+        for raw, d in zip(raws, ds):
+            cols = columns(d)
+            part = rows_of(raw, d, cols)
+            ref = O.matmul_batch(t, part, X[:active], len(cols), n)
+            old = base[:active, at + cols]
+            delta = got[:active, at + cols] - (old if residual else 0.0)
+            mag = magnitude(t, part, X[:active], len(cols), n) + (np.abs(old) * 1e-4 if residual else 0.0)
+            assert rel_err(delta, ref, mag) < F16_BOUND
+            at += d
+    proj.workspace.free()
+    for w in ws:
+        w.free()
+
+
+def test_output_columns_off_the_vector_width(ctx):
+    """An output that starts at an odd column of longer rows (no 16-byte stores), neighbours untouched."""
+    from jitllm_amd import _lib as L, synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    t, n, d, rows, ldo, off = O.Q4_0, 256, 100, 70, 131, 3
+    say("decode in registers, odd columns")
+    raw = synthetic.weight(t, d, n, seed=7120)
+    w = ctx.load_weight(t, raw, d, n)
+    X = synthetic.activations((rows, n), seed=7121)
+    proj = QuantizedBatchProjections(ctx, rows, n, d)
+    out = ctx.float_array(rows * ldo, fill=UNTOUCHED)
+    x = ctx.from_numpy(X)
+    proj._gemm([w], x, out, rows, ldo, off, L.JL_STORE)
+    ctx.sync()
+    got = out.get().reshape(rows, ldo)
+    assert np.all(got[:, :off] == UNTOUCHED) and np.all(got[:, off + d:] == UNTOUCHED)
+    assert rel_err(got[:, off:off + d], O.matmul_batch(t, raw, X, d, n), magnitude(t, raw, X, d, n)) < F16_BOUND
+    # rows of very different magnitudes: the row scale keeps each row's bits
+    Y = X * np.exp2(np.linspace(-90, 90, rows)).astype(np.float32)[:, None]
+    y = ctx.from_numpy(Y)
+    proj._gemm([w], y, out, rows, ldo, off, L.JL_STORE)
+    ctx.sync()
+    got = out.get().reshape(rows, ldo)[:, off:off + d]
+    assert rel_err(got, O.matmul_batch(t, raw, Y, d, n), magnitude(t, raw, Y, d, n)) < F16_BOUND
+    proj.workspace.free()
+    w.free()
