@@ -99,70 +99,88 @@ __device__ __forceinline__ void jl_store4_f16(_Float16 *dst, const float (&v)[4]
     }
 }
 
+// Maximum over the 64 lanes, in every lane: rotations within the rows of 16, then the halves and quarters
+// of the wave swapped (a shuffle through LDS per step took six dependent LDS round trips).
+__device__ __forceinline__ float jl_wave_max(float v) {
+#define JL_ROR(x, N) __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, x), 0x120 + N, 0xF, 0xF, false))
+    v = fmaxf(v, JL_ROR(v, 8));
+    v = fmaxf(v, JL_ROR(v, 4));
+    v = fmaxf(v, JL_ROR(v, 2));
+    v = fmaxf(v, JL_ROR(v, 1));
+#undef JL_ROR
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    v = fmaxf(__uint_as_float(h[0]), __uint_as_float(h[1]));
+    const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(v), __float_as_uint(v), false, false);
+    return fmaxf(__uint_as_float(f[0]), __uint_as_float(f[1]));
+}
+
 // Activations, fp32 -> fp16 with a power-of-two row scale.  One workgroup of 256 threads per row:
 // scale = the power of two that brings the row's largest magnitude into [2^11, 2^12);
 // a16 = half(x / scale) (the division is exact).  Rows past `rows` are zero-filled.
-// A row of up to 8192 columns is read once and kept in registers between the two passes (largest
-// magnitude, conversion); longer rows are read twice.
-__device__ __forceinline__ void jl_row_to_f16(const float *__restrict__ X, _Float16 *__restrict__ A,
-                                              float *__restrict__ row_scale, int rows, int k, int row) {
+// The first HELD x 1024 columns are read once and kept in registers between the two passes (largest
+// magnitude, conversion), what a longer row has behind them is read twice.  Every load goes out before
+// the first value is used, a pass past the row's end re-reads the thread's first columns: under a condition
+// each the loads waited for one another, and without the asm the compiler reads a value again rather
+// than keep it.
+template <int HELD>
+__device__ __forceinline__ void jl_row_to_f16_held(const float *__restrict__ x, _Float16 *__restrict__ a,
+                                                   float *__restrict__ row_scale, int k) {
     typedef _Float16 jl_half4 __attribute__((ext_vector_type(4)));
+    typedef float jl_float4 __attribute__((ext_vector_type(4)));
     __shared__ float wave_max[4];
-    constexpr int kHeld = 8;   // float4 per thread held in registers: 256 x 8 x 4 = 8192 columns
     const int tid = threadIdx.x;
-    _Float16 *a = A + (int64_t)row * k;
-    if (row >= rows) {
-        for (int i = tid * 4; i < k; i += 1024) *(jl_half4 *)(a + i) = jl_half4{0, 0, 0, 0};
-        if (tid == 0) row_scale[row] = 1.f;
-        return;
+    const int first = tid * 4 < k ? tid * 4 : 0;
+    jl_float4 v[HELD];
+#pragma unroll
+    for (int j = 0; j < HELD; j++) {
+        const int i = tid * 4 + j * 1024;
+        v[j] = *(const jl_float4 *)(x + (i < k ? i : first));
     }
-    const float *x = X + (int64_t)row * k;
-    const bool held = k <= kHeld * 1024;
-    float4 v[kHeld];
+#pragma unroll
+    for (int j = 0; j < HELD; j++) asm volatile("" : "+v"(v[j]));
+    auto largest = [](const jl_float4 &w) { return fmaxf(fmaxf(fabsf(w[0]), fabsf(w[1])), fmaxf(fabsf(w[2]), fabsf(w[3]))); };
     float amax = 0.f;
-    if (held) {
 #pragma unroll
-        for (int j = 0; j < kHeld; j++) {
-            const int i = tid * 4 + j * 1024;
-            v[j] = i < k ? *(const float4 *)(x + i) : float4{0.f, 0.f, 0.f, 0.f};
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(v[j].x), fabsf(v[j].y)), fmaxf(fabsf(v[j].z), fabsf(v[j].w))));
-        }
-    } else {
-        for (int i = tid * 4; i < k; i += 1024) {
-            float4 w = *(const float4 *)(x + i);
-            amax = fmaxf(amax, fmaxf(fmaxf(fabsf(w.x), fabsf(w.y)), fmaxf(fabsf(w.z), fabsf(w.w))));
-        }
-    }
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) amax = fmaxf(amax, __shfl_xor(amax, off, JL_WAVE));
+    for (int j = 0; j < HELD; j++) amax = fmaxf(amax, largest(v[j]));
+    for (int i = tid * 4 + HELD * 1024; i < k; i += 1024) amax = fmaxf(amax, largest(*(const jl_float4 *)(x + i)));
+    amax = jl_wave_max(amax);
     if ((tid & 63) == 0) wave_max[tid >> 6] = amax;
     __syncthreads();
     amax = fmaxf(fmaxf(wave_max[0], wave_max[1]), fmaxf(wave_max[2], wave_max[3]));
     // Every row is brought to [2^11, 2^12) at its largest magnitude: huge rows stay finite in
     // fp16, tiny rows keep their bits out of fp16's subnormal range, and the power of two is
-    // undone exactly in the epilogue.
+    // undone exactly in the epilogue.  (amax = f 2^e with f in [0.5, 1): e = its exponent field - 126,
+    // not below -100; a row of zeros, infinities or NaN alone keeps its values)
     float scale = 1.f, inv = 1.f;
     if (amax > 0.f && amax < INFINITY) {
-        int e;
-        frexpf(amax, &e);  // amax = f * 2^e, f in [0.5, 1)
+        int e = (int)(__float_as_uint(amax) >> 23) - 126;
         e = e < -100 ? -100 : e;
-        scale = ldexpf(1.f, e - 12);
-        inv = ldexpf(1.f, 12 - e);
+        scale = __uint_as_float((uint32_t)(e - 12 + 127) << 23);
+        inv = __uint_as_float((uint32_t)(12 - e + 127) << 23);
     }
-    if (held) {
+    auto put = [&](int i, const jl_float4 &w) {
+        *(jl_half4 *)(a + i) = jl_half4{(_Float16)(w[0] * inv), (_Float16)(w[1] * inv), (_Float16)(w[2] * inv), (_Float16)(w[3] * inv)};
+    };
 #pragma unroll
-        for (int j = 0; j < kHeld; j++) {
-            const int i = tid * 4 + j * 1024;
-            if (i < k)
-                *(jl_half4 *)(a + i) = jl_half4{(_Float16)(v[j].x * inv), (_Float16)(v[j].y * inv),
-                                          (_Float16)(v[j].z * inv), (_Float16)(v[j].w * inv)};
-        }
-    } else {
-        for (int i = tid * 4; i < k; i += 1024) {
-            float4 w = *(const float4 *)(x + i);
-            *(jl_half4 *)(a + i) = jl_half4{(_Float16)(w.x * inv), (_Float16)(w.y * inv), (_Float16)(w.z * inv),
-                                      (_Float16)(w.w * inv)};
-        }
+    for (int j = 0; j < HELD; j++) {
+        const int i = tid * 4 + j * 1024;
+        if (i < k) put(i, v[j]);
     }
-    if (tid == 0) row_scale[row] = scale;
+    for (int i = tid * 4 + HELD * 1024; i < k; i += 1024) put(i, *(const jl_float4 *)(x + i));
+    if (tid == 0) *row_scale = scale;
+}
+
+__device__ __forceinline__ void jl_row_to_f16(const float *__restrict__ X, _Float16 *__restrict__ A,
+                                              float *__restrict__ row_scale, int rows, int k, int row) {
+    typedef _Float16 jl_half4 __attribute__((ext_vector_type(4)));
+    _Float16 *a = A + (int64_t)row * k;
+    if (row >= rows) {
+        for (int i = threadIdx.x * 4; i < k; i += 1024) *(jl_half4 *)(a + i) = jl_half4{0, 0, 0, 0};
+        if (threadIdx.x == 0) row_scale[row] = 1.f;
+        return;
+    }
+    const float *x = X + (int64_t)row * k;
+    if (k <= 2048) jl_row_to_f16_held<2>(x, a, row_scale + row, k);
+    else if (k <= 4096) jl_row_to_f16_held<4>(x, a, row_scale + row, k);
+    else jl_row_to_f16_held<8>(x, a, row_scale + row, k);
 }
