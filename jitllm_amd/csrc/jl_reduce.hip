@@ -445,13 +445,24 @@ jl_rms_apply_f16_kernel(float *__restrict__ X, const float *__restrict__ delta, 
             ss = __fadd_rn(ss, jl_mul_rn(xi, xi));
         }
     }
+    // The reference's tree over the 256 partial sums, 128 apart first, then 64, 32, ...: the first two steps
+    // are three additions of four partial sums in every lane of every wave, the others exchanges within the
+    // wave -- one barrier instead of nine, and every thread ends with the sum.
     partial[tid] = ss;
     __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (tid < s) partial[tid] = __fadd_rn(partial[tid], partial[tid + s]);
-        __syncthreads();
-    }
-    const float m = __fadd_rn(__fdiv_rn(partial[0], (float)n), eps);
+    const int l = tid & 63;
+    float sum = __fadd_rn(__fadd_rn(partial[l], partial[l + 128]), __fadd_rn(partial[l + 64], partial[l + 192]));
+    const auto f = __builtin_amdgcn_permlane32_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __fadd_rn(__uint_as_float(f[0]), __uint_as_float(f[1]));
+    const auto h = __builtin_amdgcn_permlane16_swap(__float_as_uint(sum), __float_as_uint(sum), false, false);
+    sum = __fadd_rn(__uint_as_float(h[0]), __uint_as_float(h[1]));
+#define JL_ADD_ROR(N) sum = __fadd_rn(sum, __builtin_bit_cast(float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, sum), 0x120 + N, 0xF, 0xF, false)))
+    JL_ADD_ROR(8);
+    JL_ADD_ROR(4);
+    JL_ADD_ROR(2);
+    JL_ADD_ROR(1);
+#undef JL_ADD_ROR
+    const float m = __fadd_rn(__fdiv_rn(sum, (float)n), eps);
     // (the square root through double: correctly rounded to fp32, which __fsqrt_rn is not here)
     const float scale = __fdiv_rn(1.0f, (float)sqrt((double)m));
     if (tid == 0 && scales) scales[blockIdx.x] = scale;
