@@ -599,7 +599,10 @@ int launch_reg(jl_context *ctx, const RegParams &p) {
 // The tilings and what they cost, in microseconds a step (measured with every compute unit at work, and
 // with half of the places of the chip filled, at 2 048 and 8 192 columns, weights from HBM) and beside the
 // steps (launch, first stage, last stores).  Tilings of four waves have two workgroups to a compute unit,
-// so that half of the places is one workgroup on each.
+// so that half of the places is one workgroup on each.  Five and six row blocks are there for the row counts
+// just past 64, 128 and 256, where eight or seven leave a third of their rows empty or the chip two thirds
+// full (Q8_0 gate/up 2 x [13824 x 5120] at 65 rows 111 -> 53 us, Q4_0 q | k | v 7168 x 5120 at 270 rows 65 ->
+// 38); four row blocks with eight waves a set and two with four were never the cheapest.
 struct Tiling {
     int mb, wn, kw, places;          // places: workgroups a compute unit holds
     float base;
@@ -608,11 +611,15 @@ struct Tiling {
 constexpr Tiling kTilings[] = {
     {8, 8, 1, 1, 11.f, {2.48f, 2.05f, 2.11f, 0.f}, {1.90f, 1.53f, 1.45f, 0.f}},
     {7, 8, 1, 1, 9.f, {2.29f, 1.96f, 1.92f, 0.f}, {1.80f, 1.49f, 1.39f, 0.f}},
+    {6, 8, 1, 1, 8.5f, {2.15f, 1.87f, 1.71f, 0.f}, {1.68f, 1.42f, 1.23f, 0.f}},
+    {5, 8, 1, 1, 8.5f, {2.03f, 1.67f, 1.60f, 0.f}, {1.58f, 1.27f, 1.16f, 0.f}},
     {7, 4, 2, 1, 8.f, {0.f, 2.08f, 2.00f, 0.f}, {0.f, 1.69f, 1.66f, 0.f}},
+    {6, 4, 2, 1, 8.f, {0.f, 1.98f, 1.90f, 0.f}, {0.f, 1.65f, 1.55f, 0.f}},
+    {5, 4, 2, 1, 8.f, {2.27f, 1.86f, 1.80f, 0.f}, {1.93f, 1.55f, 1.50f, 0.f}},
     {4, 4, 2, 1, 7.f, {2.09f, 1.54f, 1.55f, 2.17f}, {1.88f, 1.34f, 1.28f, 2.14f}},
     {4, 4, 1, 2, 7.f, {1.95f, 1.60f, 1.50f, 2.13f}, {0.99f, 0.83f, 0.82f, 1.12f}},
     {4, 2, 2, 2, 6.f, {2.26f, 1.90f, 1.83f, 2.35f}, {1.14f, 0.90f, 0.86f, 1.24f}},
-    {2, 2, 2, 2, 5.f, {1.61f, 1.20f, 1.20f, 1.75f}, {0.99f, 0.70f, 0.70f, 1.15f}},
+    {2, 2, 2, 2, 5.f, {1.61f, 1.20f, 0.f, 1.75f}, {0.99f, 0.70f, 0.f, 1.15f}},
 };
 constexpr int kTilingCount = sizeof(kTilings) / sizeof(kTilings[0]);
 int type_column(int type) { return type == JL_Q8_0 ? 0 : type == JL_Q4_0 ? 1 : type == JL_Q4_K ? 2 : type == JL_Q6_K ? 3 : -1; }

@@ -34,23 +34,29 @@ def rows_of(raw, d, cols):
     return np.ascontiguousarray(raw.reshape(d, -1)[cols]).reshape(-1)
 
 
-# (type, columns, weight rows side by side, activation rows, active, gate/up, residual): the 8 x 8, 7 x 8,
-# 7 x 4 x 2, 4 x 4 x 2, 4 x 4, 4 x 2 x 2 and 2 x 2 x 2 tilings of Q4_0, then what the other types have of
-# them, as the kernel's price list chooses (a kernel trace of this file shows every instance); one block of columns (a set of waves idle), odd block counts, rows of one group, weights whose
-# last group overlaps the one before
+# (type, columns, weight rows side by side, activation rows, active, gate/up, residual): every tiling of
+# every type, as the kernel's price list chooses them (a kernel trace of this file shows each instance);
+# one block of columns (a set of waves idle), odd block counts, rows of one group, weights whose last group
+# overlaps the one before
 CASES = [
-    (O.Q4_0, 256, (14003, 14003), 449, 449, True, False), (O.Q4_0, 256, (10001, 10001), 257, 257, True, False),
+    (O.Q4_0, 512, (14003,), 449, 449, False, False), (O.Q4_0, 256, (14003, 14003), 200, 200, True, False),
+    (O.Q4_0, 256, (10001, 10001), 257, 257, True, False), (O.Q4_0, 256, (14003, 14003), 449, 449, True, False),
+    (O.Q4_0, 512, (14003, 14003), 97, 97, True, False), (O.Q4_0, 512, (14003, 14003), 81, 81, True, False),
     (O.Q4_0, 512, (14003, 14003), 65, 65, True, False), (O.Q4_0, 512, (5005,), 300, 300, False, True),
     (O.Q4_0, 256, (14003, 14003), 97, 97, True, False), (O.Q4_0, 512, (10001,), 129, 129, False, False),
     (O.Q4_0, 256, (16,), 65, 65, False, True), (O.Q4_0, 256, (100, 17, 33), 65, 65, False, True),
+    (O.Q8_0, 512, (14003,), 449, 449, False, False), (O.Q8_0, 256, (14003, 14003), 200, 200, True, False),
     (O.Q8_0, 256, (14003, 14003), 449, 449, True, False), (O.Q8_0, 256, (10001, 10001), 257, 257, True, False),
+    (O.Q8_0, 512, (14003, 14003), 65, 65, True, False),
     (O.Q8_0, 512, (12001,), 257, 257, False, True), (O.Q8_0, 256, (12001, 12001), 200, 199, True, False),
     (O.Q8_0, 512, (3003, 3003), 257, 257, True, False), (O.Q8_0, 512, (3003, 17, 100), 65, 65, False, False),
-    (O.Q4_K, 512, (14003, 14003), 449, 449, True, False), (O.Q4_K, 2304, (16390, 16390), 65, 65, True, False),
-    (O.Q4_K, 2816, (8200, 8200), 97, 97, True, False), (O.Q4_K, 2816, (2050, 2050), 384, 384, True, False),
-    (O.Q4_K, 2304, (6007, 6007), 257, 257, True, False), (O.Q4_K, 2816, (1002, 1002), 449, 440, True, False),
+    (O.Q4_K, 512, (14003, 14003), 511, 511, True, False), (O.Q4_K, 1280, (12001, 12001), 200, 200, True, False),
+    (O.Q4_K, 512, (12001, 12001), 449, 449, True, False), (O.Q4_K, 2304, (16390, 16390), 65, 65, True, False),
+    (O.Q4_K, 2816, (8200, 8200), 97, 97, True, False), (O.Q4_K, 2304, (4099, 4099), 255, 255, True, False),
+    (O.Q4_K, 2304, (4099, 4099), 240, 240, True, False), (O.Q4_K, 2816, (2050, 2050), 384, 384, True, False),
+    (O.Q4_K, 2816, (5005, 5005), 161, 161, True, False), (O.Q4_K, 2816, (1002, 1002), 449, 440, True, False),
     (O.Q6_K, 5888, (5005,), 200, 200, False, True),
-    (O.Q6_K, 256, (33,), 128, 128, False, True), (O.Q6_K, 512, (4099,), 128, 128, False, False),
+    (O.Q6_K, 256, (33,), 128, 128, False, True), (O.Q6_K, 512, (4099,), 161, 161, False, False),
     (O.Q6_K, 768, (4099, 4099), 128, 128, True, False), (O.Q6_K, 2816, (40, 17), 140, 130, False, False),
     (O.Q6_K, 768, (100, 100), 160, 145, True, False),
 ]
