@@ -247,8 +247,9 @@ int jl_argmax_rows(jl_context *ctx, const float *values, int64_t rows, int64_t n
  * there), x used as it is when rms_weights is null -- and index[0] = jl_argmax(out) (the
  * vocabulary projection followed by "argmax_sample", LogitsQ8_0Layer.java:92-110,
  * LogitsFP16Layer.java:217).  out and index[0] are bit for bit what jl_gemv / jl_gemv_rms followed
- * by jl_argmax leave.  A Q8_0, Q4_0 or Q4_K weight of 2048 or 4096 columns and a multiple of eight
- * (four) rows takes two launches instead of three: the projection's workgroups keep the largest
+ * by jl_argmax leave.  A Q8_0, Q4_0 or Q4_K weight of 513 ... 4096 columns (a multiple of 64) and whole
+ * tiles of rows (a multiple of 16 up to 1024 columns, of eight up to 2048, of four beyond), spread over
+ * at most 1024 workgroups, takes two launches instead of three: the projection's workgroups keep the largest
  * logit they store and its row, and the second launch folds those thousand candidates instead of
  * reading the logits back.  Any other weight the single-token kernels take is the two calls, made
  * here.

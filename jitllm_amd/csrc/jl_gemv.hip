@@ -786,7 +786,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     constexpr bool FULL = LEAN && !PART;   // every lane has a slice, every load slot is real data
     static_assert(!PART || LEAN, "rows shorter than SPT slices: a fixed tile shape");
     static_assert(!LEAN || !PACKED, "the packed form has no fixed-geometry instances");
-    static_assert(!ARGMAX || (FULL && !DUAL && !SEGS && SPT <= 64), "the argmax form: whole in-wave rows of one weight");
+    static_assert(!ARGMAX || (LEAN && !DUAL && !SEGS && SPT <= 64), "the argmax form: in-wave rows of one weight");
     static_assert(!HALVES || (PART && !DUAL && !RMS && !PACKED && !SEGS && !ARGMAX && THREADS == 1024 && SPT == 256),
                   "rows in two halves: the plain 1024-thread form");
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -1424,6 +1424,17 @@ int launch_fixed(jl_context *ctx, const GemvParams &p, int lds, bool full) {
     }
 }
 
+// The argmax form of a plain or RMS-folding projection with rows padded to SP slices.
+template <int TYPE, int SP>
+int launch_argmax(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
+    if (p.S == p.Sp) {
+        return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells)
+                       : launch_tiles_of<TYPE, false, false, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells);
+    }
+    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells)
+                   : launch_tiles_of<TYPE, false, false, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells);
+}
+
 // `fixed`: the launch meets the fixed-geometry form's conditions (whole tiles only in every
 // weight).  The three main types have an instance for every variant at row lengths of 513 ... 8192
 // columns and, in the 1024-thread form (plain and residual), up to 16384 -- and, a row taken as two
@@ -1435,16 +1446,18 @@ int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, boo
     // (side types: plain, residual and gate/up only -- the caller has refused the rest)
     constexpr bool kMain = is_main_type(TYPE);
     if (cells) {
-        // the argmax form: one main-type weight, whole tiles of whole in-wave rows of 2048 or 4096
-        // columns, stored (not accumulated) outputs
+        // the argmax form: one main-type weight, whole tiles of in-wave rows (513 ... 4096 columns), stored (not
+        // accumulated) outputs.  Elsewhere the logits are scanned in a launch of their own: 151936 x 896 Q8_0 with
+        // its argmax 35.1 us with the scan, 31.8 with cells (a token of that model 435 -> 426 us).  Q6_K on its
+        // fixed-geometry instances gained nothing (a token with a 152064 x 3584 vocabulary 1503 and 1504 us).
         if constexpr (kMain && !DUAL) {
-            if (fixed && threads == 256 && p.S == p.Sp && p.nseg == 1 && !p.xq && p.epilogue == JL_STORE) {
-                if (p.Sp == 32)
-                    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, 32, false, false, true>(ctx, p, 256, lds, cells)
-                                   : launch_tiles_of<TYPE, false, false, false, 256, 32, false, false, true>(ctx, p, 256, lds, cells);
-                if (p.Sp == 64)
-                    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, 64, false, false, true>(ctx, p, 256, lds, cells)
-                                   : launch_tiles_of<TYPE, false, false, false, 256, 64, false, false, true>(ctx, p, 256, lds, cells);
+            if (fixed && threads == 256 && p.nseg == 1 && !p.xq && p.epilogue == JL_STORE) {
+                switch (p.Sp) {
+                    case 16: return launch_argmax<TYPE, 16>(ctx, p, lds, cells);
+                    case 32: return launch_argmax<TYPE, 32>(ctx, p, lds, cells);
+                    case 64: return launch_argmax<TYPE, 64>(ctx, p, lds, cells);
+                    default: break;
+                }
             }
         }
         return JL_NO_CELLS_FORM;

@@ -217,12 +217,24 @@ __global__ void __launch_bounds__(kArgmaxThreads) jl_argmax_fold_cells(const flo
     __shared__ float pv[kArgmaxThreads / JL_WAVE];
     __shared__ int pi[kArgmaxThreads / JL_WAVE];
     const int tid = threadIdx.x;
+    const float first = values[0];   // asked for with the cells: read behind the fold it is one more trip to memory
     float best = -INFINITY;
     int at = INT_MAX;
-    for (int i = tid; i < cells; i += kArgmaxThreads) keep_better(best, at, cell_value[i], cell_index[i]);
+    // (all of a thread's cells, at most four, in one trip)
+    constexpr int kEach = (kProjectionCells + kArgmaxThreads - 1) / kArgmaxThreads;
+    float v[kEach];
+    int r[kEach];
+#pragma unroll
+    for (int j = 0; j < kEach; j++) {
+        const int i = tid + j * kArgmaxThreads < cells ? tid + j * kArgmaxThreads : 0;
+        v[j] = cell_value[i];
+        r[j] = cell_index[i];
+    }
+#pragma unroll
+    for (int j = 0; j < kEach; j++) keep_better(best, at, v[j], r[j]);
     fold_waves(best, at, pv, pi, tid, kArgmaxThreads / JL_WAVE);
     if (tid == 0) {
-        if (at == INT_MAX || values[0] != values[0]) at = 0;   // as in jl_argmax_fold
+        if (at == INT_MAX || first != first) at = 0;   // as in jl_argmax_fold
         index[0] = at;
     }
 }

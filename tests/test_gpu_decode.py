@@ -609,9 +609,9 @@ def test_rms_vocabulary_projection_and_argmax(ctx, t, d, n):
     assert rel_err(logits.get(), ref, magnitude(t, raw, xn, d, n)) < 2e-5
 
 
-# (type, rows, columns): the first four take the projection kernel that keeps its workgroups' best
-# logits; then a row count that is not whole tiles, rows shorter than their padded slices, rows in
-# several waves, a type with no such form -- those run the projection and the scan, inside the call
+# (type, rows, columns): the first four and the rows shorter than their padded slices take the
+# projection kernel that keeps its workgroups' best logits; a row count that is not whole tiles, rows
+# in several waves, a type with no such form run the projection and the scan, inside the call
 PROJECTION_ARGMAX = [(O.Q8_0, 32000, 2048), (O.Q4_0, 20008, 4096), (O.Q4_K, 16384, 2048), (O.Q4_K, 4100, 4096),
                      (O.Q8_0, 1001, 2048), (O.Q8_0, 9000, 3072), (O.Q4_0, 3000, 8192), (O.Q6_K, 5000, 2048)]
 
@@ -663,6 +663,16 @@ def test_projection_and_argmax_in_one_call(ctx, t, d, n, rms):
     assert bits_equal(got, want)
     assert got_token == want_token == O.argmax(want)
     assert np.count_nonzero(want == want[want_token]) >= 2 and want_token == int(np.flatnonzero(want == want.max())[0])
+
+
+# one tile, many, and a workgroup's first and last rows, of rows of fewer slices than their lanes (and of 16
+# slices, whole)
+@pytest.mark.parametrize("t,d,n", [(O.Q8_0, 16, 896), (O.Q8_0, 40000, 896), (O.Q4_0, 4096, 640), (O.Q4_K, 4112, 1024),
+                                   (O.Q4_0, 5000, 1536), (O.Q4_K, 9004, 3584)])
+@pytest.mark.parametrize("rms", ["plain", "scale given", "scale in kernel"])
+def test_projection_and_argmax_of_short_rows(ctx, t, d, n, rms):
+    """The further shapes whose projection keeps the best logits: as in the test above."""
+    test_projection_and_argmax_in_one_call(ctx, t, d, n, rms)
 
 
 @pytest.mark.parametrize("t,d,n", [(O.Q8_0, 32000, 2048), (O.Q4_K, 4100, 4096)])
