@@ -23,8 +23,8 @@
 // What bounds it: at MB = 8 a step issues 64 matrix instructions, 1 024 cycles a wave, two waves to a SIMD; LDS
 // (8 waves x 32 KB of activations), vector instructions and loads take about half of those cycles each,
 // and the parts hide each other by half: 41 % of the matrix rate at the clock it runs at (rocprofv3:
-// SQ_VALU_MFMA_BUSY_CYCLES against SQ_BUSY_CYCLES).  Without the raw bytes' way a step is a fifth shorter,
-// without the decode a tenth, without either and the stage loads a third.
+// SQ_VALU_MFMA_BUSY_CYCLES against SQ_BUSY_CYCLES).  Without the raw bytes' way a launch is a sixth
+// shorter, without the decode a tenth, without either and the stage loads a third.
 // Measured (one box, weights from HBM, before -> now): Q4_K gate/up 2 x [11008 x 4096] at 201 rows 107 -> 55
 // us, q | k | v 12288 x 4096 61 -> 37, Q4_0 gate/up 2 x [14592 x 4096] at 99 rows 53 -> 43, Q8_0 q | k | v
 // 13824 x 4608 at 408 rows 123 -> 84, Q6_K 4096 x 14336 at 256 rows 127 -> 79.

@@ -1424,17 +1424,6 @@ int launch_fixed(jl_context *ctx, const GemvParams &p, int lds, bool full) {
     }
 }
 
-// The argmax form of a plain or RMS-folding projection with rows padded to SP slices.
-template <int TYPE, int SP>
-int launch_argmax(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
-    if (p.S == p.Sp) {
-        return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells)
-                       : launch_tiles_of<TYPE, false, false, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells);
-    }
-    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells)
-                   : launch_tiles_of<TYPE, false, false, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells);
-}
-
 // `fixed`: the launch meets the fixed-geometry form's conditions (whole tiles only in every
 // weight).  The three main types have an instance for every variant at row lengths of 513 ... 8192
 // columns and, in the 1024-thread form (plain and residual), up to 16384 -- and, a row taken as two
@@ -1442,26 +1431,9 @@ int launch_argmax(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
 // 2048, 4096 and (plain and residual) 8192 columns, Q6_K also for plain and residual rows of 2304 ... 3840
 // columns and, as two half rows, of 16896 ... 32768.
 template <int TYPE, bool DUAL>
-int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed, int *cells = nullptr) {
+int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed) {
     // (side types: plain, residual and gate/up only -- the caller has refused the rest)
     constexpr bool kMain = is_main_type(TYPE);
-    if (cells) {
-        // the argmax form: one main-type weight, whole tiles of in-wave rows (513 ... 4096 columns), stored (not
-        // accumulated) outputs.  Elsewhere the logits are scanned in a launch of their own: 151936 x 896 Q8_0 with
-        // its argmax 35.1 us with the scan, 31.8 with cells (a token of that model 435 -> 426 us).  Q6_K on its
-        // fixed-geometry instances gained nothing (a token with a 152064 x 3584 vocabulary 1503 and 1504 us).
-        if constexpr (kMain && !DUAL) {
-            if (fixed && threads == 256 && p.nseg == 1 && !p.xq && p.epilogue == JL_STORE) {
-                switch (p.Sp) {
-                    case 16: return launch_argmax<TYPE, 16>(ctx, p, lds, cells);
-                    case 32: return launch_argmax<TYPE, 32>(ctx, p, lds, cells);
-                    case 64: return launch_argmax<TYPE, 64>(ctx, p, lds, cells);
-                    default: break;
-                }
-            }
-        }
-        return JL_NO_CELLS_FORM;
-    }
     if constexpr (kMain) {
         if (p.xq) return launch_tiles_of<TYPE, DUAL, false, true>(ctx, p, threads, lds);
     }
@@ -1508,6 +1480,9 @@ int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, boo
     }
     return launch_tiles_of<TYPE, DUAL, false>(ctx, p, threads, lds);
 }
+
+// the argmax form of a projection, below
+int launch_argmax_of(jl_context *ctx, const GemvParams &p, int type, int threads, int lds, bool fixed, int *cells);
 
 template <int TYPE>
 int launch_generic(jl_context *ctx, const jl_weight *w, const jl_weight *w_up, const float *x,
@@ -1686,13 +1661,8 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     for (int i = 0; i < nseg; i++) fixed = fixed && w[i]->rows % half_rows == 0;
 
     if (cells) {
-        if (dual) return JL_NO_CELLS_FORM;
-        switch (type) {
-            case JL_Q8_0: return launch_tiles<JL_Q8_0, false>(ctx, p, threads, lds, fixed, &cells->count);
-            case JL_Q4_0: return launch_tiles<JL_Q4_0, false>(ctx, p, threads, lds, fixed, &cells->count);
-            case JL_Q4_K: return launch_tiles<JL_Q4_K, false>(ctx, p, threads, lds, fixed, &cells->count);
-            default: return JL_NO_CELLS_FORM;
-        }
+        if (dual || nseg != 1 || xq || epilogue != JL_STORE) return JL_NO_CELLS_FORM;
+        return launch_argmax_of(ctx, p, type, threads, lds, fixed, &cells->count);
     }
     switch (type) {
         case JL_Q8_0:
@@ -1724,3 +1694,43 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
                            "no single-token projection kernel for a ggml type %d weight", type);
     }
 }
+
+namespace {
+
+// The argmax form of a plain or RMS-folding projection with rows padded to SP slices.
+template <int TYPE, int SP>
+int launch_argmax_sp(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
+    if (p.S == p.Sp) {
+        return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells)
+                       : launch_tiles_of<TYPE, false, false, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells);
+    }
+    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells)
+                   : launch_tiles_of<TYPE, false, false, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells);
+}
+// One main-type weight, whole tiles of in-wave rows (513 ... 4096 columns), stored (not accumulated) outputs.
+// Elsewhere the logits are scanned in a launch of their own: 151936 x 896 Q8_0 with its argmax 35.1 us with the
+// scan, 31.8 with cells (a token of that model 435 -> 426 us).  Q6_K on its fixed-geometry instances gained
+// nothing (a token with a 152064 x 3584 vocabulary 1503 and 1504 us).
+template <int TYPE>
+int launch_argmax(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed, int *cells) {
+    if (fixed && threads == 256) {
+        switch (p.Sp) {
+            case 16: return launch_argmax_sp<TYPE, 16>(ctx, p, lds, cells);
+            case 32: return launch_argmax_sp<TYPE, 32>(ctx, p, lds, cells);
+            case 64: return launch_argmax_sp<TYPE, 64>(ctx, p, lds, cells);
+            default: break;
+        }
+    }
+    return JL_NO_CELLS_FORM;
+}
+
+int launch_argmax_of(jl_context *ctx, const GemvParams &p, int type, int threads, int lds, bool fixed, int *cells) {
+    switch (type) {
+        case JL_Q8_0: return launch_argmax<JL_Q8_0>(ctx, p, threads, lds, fixed, cells);
+        case JL_Q4_0: return launch_argmax<JL_Q4_0>(ctx, p, threads, lds, fixed, cells);
+        case JL_Q4_K: return launch_argmax<JL_Q4_K>(ctx, p, threads, lds, fixed, cells);
+        default: return JL_NO_CELLS_FORM;
+    }
+}
+
+}  // namespace
