@@ -1595,8 +1595,10 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     }
     if (is_side_type(type)) {
         // measured: the tile kernel is the faster one from rows of 2048 columns and 2 MB of weights
-        // (by up to 1.7 x on the vocabulary and feed-forward projections); below that the two are
-        // within a few tenths of a microsecond of each other and the one-wave-per-row kernel stays.
+        // (by up to 1.7 x on the vocabulary and feed-forward projections).  Below 2 MB the one-wave-per-row kernel stays
+        // for its error, not its time: Q6_K 512 x 3584 4.4 us here and 3.3 on the tile kernel, 512 x 4096 4.0 and 3.1,
+        // 256 x 8192 5.8 and 3.5, but rows that fill their slices only in part come out up to 2.4 % further from
+        // their float64 values (3584 columns, 2-norm: 1.514e-7 and 1.526e-7); Q5_K loses 2 - 4 % at 2304 - 3072 columns.
         // (Q6_K rows whose tiles start off a 16-byte boundary, every super-block count from 9 to 63 at 2 MB, 1024,
         // 3584, 8192 and 32768 rows: 0.44 - 0.94 of the one-wave-per-row kernel's time, also where half of a tile's
         // threads have no slice -- 17 super-blocks: 592 rows 5.05 and 4.55 us, 8192 rows 16.8 and 12.1 -- and from 61,
