@@ -1595,15 +1595,18 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
     }
     if (is_side_type(type)) {
         // measured: the tile kernel is the faster one from rows of 2048 columns and 2 MB of weights
-        // (by up to 1.7 x on the vocabulary and feed-forward projections).  Below 2 MB the one-wave-per-row kernel stays
-        // for its error, not its time: Q6_K 512 x 3584 4.4 us here and 3.3 on the tile kernel, 512 x 4096 4.0 and 3.1,
-        // 256 x 8192 5.8 and 3.5, but rows that fill their slices only in part come out up to 2.4 % further from
-        // their float64 values (3584 columns, 2-norm: 1.514e-7 and 1.526e-7); Q5_K loses 2 - 4 % at 2304 - 3072 columns.
+        // (by up to 1.7 x on the vocabulary and feed-forward projections), and below 2 MB on whole tiles of Q6_K rows that
+        // fill their slices, plain and residual: 512 x 4096 4.0 us on the one-wave-per-row kernel and 3.1 here, 256 x 8192
+        // 5.8 and 3.5, 512 x 2048 2.80 and 2.76 (48 x 2048 2.54 and 2.58: of that length from 128 KB on).  On other Q6_K rows it is the faster one too (512 x 3584 4.4 and 3.3),
+        // but up to 2.4 % further from the float64 values (3584 columns, 2-norm: 1.514e-7 and 1.526e-7; whole rows
+        // 4096 columns 1.534e-7 and 1.528e-7): those stay.  Q5_K loses 2 - 4 % at 2304 - 3072 columns.
         // (Q6_K rows whose tiles start off a 16-byte boundary, every super-block count from 9 to 63 at 2 MB, 1024,
         // 3584, 8192 and 32768 rows: 0.44 - 0.94 of the one-wave-per-row kernel's time, also where half of a tile's
         // threads have no slice -- 17 super-blocks: 592 rows 5.05 and 4.55 us, 8192 rows 16.8 and 12.1 -- and from 61,
         // whose 256 threads take one row a tile: 168 rows 9.5 and 5.3, 8192 rows 48.9 and 38.5)
-        if (!fast || n < 2048 || w[0]->bytes * (dual ? 2 : 1) < ((int64_t)2 << 20))
+        const bool whole_q6 = fast && type == JL_Q6_K && !dual && S == Sp && S <= 128 && w[0]->rows % half_rows == 0 &&
+                              (S > 32 || w[0]->bytes >= (int64_t)128 << 10);
+        if (!fast || n < 2048 || (!whole_q6 && w[0]->bytes * (dual ? 2 : 1) < ((int64_t)2 << 20)))
             return jl_launch_gemv_direct(ctx, w[0], w_up, x, outs[0], epilogue);
     }
     if (!fast) {

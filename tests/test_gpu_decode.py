@@ -914,6 +914,8 @@ def q6_k_takes_the_tile_kernel(d, n):
     row_bytes = n // 256 * 210
     if 16384 < n <= 32768 and n % 512 == 0 and d % 2 == 0 and d * row_bytes % 16 == 0:
         return True
+    if n in (2048, 4096, 8192) and d % (16384 // n) == 0 and (n > 2048 or d * row_bytes >= 128 << 10):
+        return True
     return 2048 <= n <= 16384 and d * row_bytes % 16 == 0 and d * row_bytes >= 2 << 20
 
 
@@ -983,6 +985,38 @@ def test_q6_k_fixed_geometry_and_general_instances_give_the_same_bits(ctx, d, n)
         ctx.sync()
         got.append(out.get())
     assert np.all(got[1] != POISON) and bits_equal(got[0], got[1][:d])
+
+
+@pytest.mark.parametrize("d,n", [(80, 2048), (88, 2048), (1240, 2048), (4, 4096), (512, 4096), (2, 8192), (256, 8192), (310, 8192)])
+def test_q6_k_small_weights_of_whole_slices(ctx, d, n):
+    """Less than 2 MB in whole tiles of rows of 32, 64 or 128 slices, from one tile (of 2048 columns: from 128 KB) on: the bits of the same rows
+    inside a larger weight (the tile kernel's at every size), plain and residual, and the oracle's sums to 2e-5 of
+    their magnitude as everywhere; nothing behind the last row is touched."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedProjections, TornadoWorkspace
+    say("q6_k small", d, n)
+    large = 8 * (-(-(2 << 20) // (n // 256 * 210 * 8)))
+    assert q6_k_takes_the_tile_kernel(large, n) and d < large
+    raw = np.asarray(synthetic.weight(O.Q6_K, large, n, seed=7960)).reshape(large, -1)
+    x = synthetic.activations(n, seed=7961)
+    base = synthetic.activations(large, seed=7962)
+    dx = ctx.from_numpy(x)
+    got = []
+    for rows in (d, large):
+        w = upload(ctx, O.Q6_K, raw[:rows].reshape(-1), rows, n)
+        out = ctx.float_array(rows + 8, fill=POISON)
+        acc = ctx.from_numpy(base.copy())
+        proj = QuantizedProjections(ctx, TornadoWorkspace(wrapX=acc))
+        proj.floatMatvec(dx, out, w, n, rows)
+        proj.residualMatvec(dx, w, n, rows)
+        ctx.sync()
+        got.append((out.get(), acc.get()))
+        w.free()
+    (small, added), (whole, added_whole) = got
+    assert np.all(small[d:] == POISON) and bits_equal(added[d:], base[d:])
+    assert bits_equal(small[:d], whole[:d]) and bits_equal(added[:d], added_whole[:d])
+    ref = O.matmul(O.Q6_K, raw[:d].reshape(-1), x, d, n)
+    assert rel_err(small[:d], ref, magnitude(O.Q6_K, raw[:d].reshape(-1), x, d, n)) < 2e-5
 
 
 @pytest.mark.parametrize("d,n", [(1200, 2304), (1024, 3584), (256, 11008), (16, 18944)])
