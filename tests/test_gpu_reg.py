@@ -139,3 +139,34 @@ def test_output_columns_off_the_vector_width(ctx):
     assert rel_err(got, O.matmul_batch(t, raw, Y, d, n), magnitude(t, raw, Y, d, n)) < F16_BOUND
     proj.workspace.free()
     w.free()
+
+
+# columns, weight rows, activation rows of Q6_K calls that the streaming kernel would take were they not cheaper here
+@pytest.mark.parametrize("n,d,rows", [(4096, 4096, 384), (8192, 4096, 511), (14336, 4096, 256)])
+def test_q6_k_sums_are_as_exact_as_the_streaming_kernels(ctx, n, d, rows):
+    """Weights that no kernel rounds (|scale x quant| <= 2048) and binary16 activations: all of the error against
+    float64 is that of the fp32 sums.  The same rows in a call of 64, which the weight-streaming kernel takes,
+    are the measure: 12 800 values tell its error to 0.6 % (one over the root of twice as many), 3 % is five
+    times that.  (Added result by result this kernel's sums are 4, 20 and 39 % further off.)"""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("decode in registers, q6_k sums", n, d, rows)
+    raw = np.array(synthetic.weight(O.Q6_K, d, n, seed=7130)).reshape(-1, 210)
+    raw[:, 192:208] = (raw[:, 192:208].view(np.int8) >> 1).view(np.uint8)
+    X = synthetic.activations((rows, n), seed=7131).astype(np.float16)
+    w = ctx.load_weight(O.Q6_K, raw.reshape(-1), d, n)
+    x = ctx.half_from_numpy(X)
+    proj = QuantizedBatchProjections(ctx, rows, n, d)
+    cols = np.arange(7, d, d // 200)[:200]
+    exact = X.astype(np.float64) @ O.dequant(O.Q6_K, rows_of(raw.reshape(-1), d, cols)).reshape(len(cols), n).astype(np.float64).T
+    err = []
+    for active in (64, rows):
+        out = ctx.float_array(rows * d)
+        proj.projection(x, out, w, n, d, False, active)
+        ctx.sync()
+        got = out.get().reshape(rows, d)[:active, cols].astype(np.float64)
+        err.append(np.linalg.norm(got - exact[:active]) / np.linalg.norm(exact[:active]))
+    print("error, streaming kernel %.4e, in registers %.4e" % tuple(err))
+    assert err[1] <= 1.03 * err[0], err
+    proj.workspace.free()
+    w.free()
