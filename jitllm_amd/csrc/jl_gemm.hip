@@ -972,33 +972,26 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     const double copy_us = kept && rows >= 128 ? 24.0 + 0.45 * ((rows + 255) / 256) * millions
                            : dense_only       ? 30.0 + 2.8 * millions
                                               : 1e30;
-    // ... and the kernel that decodes in registers, priced by its own table, at 65 .. 511 rows.  With Q4_K it
-    // rounds a weight to fp16, as the ways that decode in the loop or once do and the weight-streaming kernel
-    // does not: of that type it takes calls from those only, after the streaming kernel has had its choice.
+    // ... and the kernel that decodes in registers, priced by its own table, at 65 .. 511 rows.  The
+    // weight-streaming kernel multiplies Q4_K and Q6_K weights unrounded and adds fewer results in a row: of
+    // those types it keeps every call that it would have without this kernel, which rounds Q4_K weights to
+    // fp16 as the other two ways do, and adds Q6_K's results in one long sum (4096 x 14336 at 256 rows 72 us
+    // instead of 120, but 1.59e-7 off float64 instead of 1.10e-7 over weights that neither rounds).  Q6_K calls
+    // that would else be decoded to fp16 become more exact here (2.0e-4 to 1.4e-4 off the float64 values).
     // A call over a kept copy gives the bits of one without from 512 rows on and below 128: it is not
     // considered from 512 on, nor where a copy is kept and read, and Q6_K (whose calls read a kept copy at any
-    // row count) comes here from 128 on.  Q6_K calls that would else be streamed, whose weights are not
-    // rounded either, it takes by tilings with sums as short only; calls that would else be decoded to fp16
-    // become more exact by any (2.1e-4 to 1.4e-4 off the float64 values).
+    // row count) comes here from 128 on.
     int reg_tiling = -1;
     double reg_us = 1e30;
-    const double decode_us = in_loop_us < copy_us ? in_loop_us : copy_us;
-    if (rows < 512 && rows >= (dense_only ? 128 : 65) && !(kept && (rows >= 128 || dense_only)) && workspace_bytes >= head) {
-        bool streams = false;
-        if (type == JL_Q6_K) {
-            const int st = jl_launch_gemm_skinny(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue,
-                                                 planes, plane_bytes, decode_us, &streams, true);
-            if (st != JL_OK) return st;
-        }
-        reg_us = jl_gemm_reg_price(ctx, weights, count, rows, epilogue, streams, &reg_tiling);
-    }
+    if (rows < 512 && rows >= (dense_only ? 128 : 65) && !(kept && (rows >= 128 || dense_only)) && workspace_bytes >= head)
+        reg_us = jl_gemm_reg_price(ctx, weights, count, rows, epilogue, &reg_tiling);
     if (rows < 512) {
         // batched decode of up to 64 rows, and calls of up to 511 where it is the cheapest: the
         // weight-streaming kernel reads X itself, fp32 or fp16
         bool taken = false;
-        double other_us = decode_us;
+        double other_us = in_loop_us < copy_us ? in_loop_us : copy_us;
         // (near equal prices the streaming kernel is the faster one, by up to 8 %, measured)
-        if (1.1 * reg_us < other_us && type != JL_Q4_K) other_us = 1.1 * reg_us;
+        if (1.1 * reg_us < other_us && type != JL_Q4_K && type != JL_Q6_K) other_us = 1.1 * reg_us;
         int st = jl_launch_gemm_skinny(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue,
                                        planes, plane_bytes, other_us, &taken);
         if (st != JL_OK || taken) return st;

@@ -27,7 +27,7 @@
 // shorter, without the decode a tenth, without either and the stage loads a third.
 // Measured (one box, weights from HBM, before -> now): Q4_K gate/up 2 x [11008 x 4096] at 201 rows 107 -> 55
 // us, q | k | v 12288 x 4096 61 -> 37, Q4_0 gate/up 2 x [14592 x 4096] at 99 rows 53 -> 43, Q8_0 q | k | v
-// 13824 x 4608 at 408 rows 123 -> 84, Q6_K 4096 x 14336 at 256 rows 127 -> 79.
+// 13824 x 4608 at 408 rows 123 -> 84, Q6_K gate/up 2 x [13824 x 5120] at 128 rows 179 -> 80.
 // Tried and taken back: activation fragments two row blocks ahead (55.2 against 56.4 us, and it spills
 // with Q8_0); three stages (no change); matrix instructions at raised priority (no change); 32-byte quant
 // runs read from LDS unaligned instead of funnel-shifted (68 against 46 us).
@@ -218,32 +218,12 @@ __device__ __forceinline__ int row_key(int row) {
 }
 
 // LDS: per set of waves two stages of activations (128 columns of 16 MB rows each), then every wave's raw
-// bytes (the last word that a lane reads may lie past them), then second-level sums (sum_places)
+// bytes (the last word that a lane reads may lie past them)
 constexpr int kStages = 2;
-constexpr int kLds = 160 * 1024;
-constexpr int ring_bytes(int type, int mb, int wn, int kw) { return kw * kStages * mb * 4096 + wn * kw * NR * raw_bytes(type) + 16; }
-constexpr int sums_bytes(int mb, int wn) { return wn * mb * NR * 1024; }
-// Q6_K weights whose scale x quant is at most 2048 are multiplied unrounded, and with fp16 activations the
-// fp32 sums are then all the error that a call has.  Added result by result (128 columns each) a row of
-// 14336 columns is 1.56e-7 off the float64 values; the weight-streaming kernel, which adds 256 columns, eight
-// waves, spans, is 1.12e-7 off.  So a running sum of Q6_K moves every four blocks to a second one in LDS (no
-// register is free for it): one for each set of waves, 1.08e-7, or where there is only room for one, the
-// sets come there in turn, 1.18e-7 (8192 columns 1.07e-7, both kernels).  Where even that would cost the
-// compute unit a workgroup the sums stay long.  (The other types' weights are rounded to fp16: 1.4e-4.)
-constexpr int sum_places(int type, int mb, int wn, int kw) {
-    const int ring = ring_bytes(type, mb, wn, kw);
-    if (type != JL_Q6_K || kw != 2) return 0;
-    return kLds / (ring + 2 * sums_bytes(mb, wn)) == kLds / ring ? 2 : kLds / (ring + sums_bytes(mb, wn)) == kLds / ring ? 1 : 0;
-}
-// the most blocks of a set whose sums are then no longer than the weight-streaming kernel's
-constexpr int short_sum_blocks(int type, int mb, int wn, int kw) {
-    const int places = sum_places(type, mb, wn, kw);
-    return type != JL_Q6_K || places == 2 ? 1 << 30 : places == 1 ? 16 : 4;
-}
 template <int TYPE, int MB, int WN, int KW> constexpr int lds_bytes() {
-    constexpr int loop = ring_bytes(TYPE, MB, WN, KW) + sum_places(TYPE, MB, WN, KW) * sums_bytes(MB, WN);
+    constexpr int ring = KW * kStages * MB * 4096 + WN * KW * NR * raw_bytes(TYPE) + 16;
     constexpr int fold = KW > 1 ? KW * WN * MB * NR * 1024 : 0;
-    return loop > fold ? loop : fold;
+    return ring > fold ? ring : fold;
 }
 
 template <int TYPE, int MB, int WN, int KW>
@@ -382,38 +362,6 @@ jl_gemm_reg(RegParams p) {
     for (int m = 0; m < MB; m++)
 #pragma unroll
         for (int j = 0; j < NR; j++) total[m][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-
-    // The second level of sums: `total` is added to that in LDS (`first`: put there) and starts again (`last`:
-    // what lies there is added to it).  Sets that share one come to it in turn, set 1 after the first pair of
-    // blocks and every second one from there, set 0 after those between: barriers lie between any two of them.
-    constexpr int SUMS = sum_places(TYPE, MB, WN, KW);
-    const uint32_t sums = lds0 + ring_bytes(TYPE, MB, WN, KW) + (SUMS == 2 ? wave : wn) * (MB * NR * 1024) + lane * 16;
-    auto move_sums = [&](bool first, bool last) {
-        if (!first) {
-#pragma unroll
-            for (int m = 0; m < MB; m++) {
-                u32x4 s[NR];
-#pragma unroll
-                for (int j = 0; j < NR; j++)
-                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(s[j]) : "v"(sums), "n"((m * NR + j) * 1024) : "memory");
-                asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-                settled(s);
-#pragma unroll
-                for (int j = 0; j < NR; j++) total[m][j] += __builtin_bit_cast(floatx4, s[j]);
-            }
-        }
-        if (last) return;
-#pragma unroll
-        for (int m = 0; m < MB; m++)
-#pragma unroll
-            for (int j = 0; j < NR; j++)
-                asm volatile("ds_write_b128 %0, %1 offset:%2" : : "v"(sums), "v"(total[m][j]), "n"((m * NR + j) * 1024) : "memory");
-        asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");
-#pragma unroll
-        for (int m = 0; m < MB; m++)
-#pragma unroll
-            for (int j = 0; j < NR; j++) total[m][j] = floatx4{0.f, 0.f, 0.f, 0.f};
-    };
 
     // slice g of the 128 columns is chunks 4 (g % 2) .. of half g / 2; fragment i of row block m lies at
     // (a_base ^ (i << 4)) + m * 2048
@@ -554,15 +502,6 @@ jl_gemm_reg(RegParams p) {
     for (int it = 0; it < iters; it += 2) {
         block(it, 0);
         if (it + 1 < iters) block(it + 1, 1);
-        if constexpr (SUMS > 0) {
-            const int turn = SUMS == 1 ? kw : 0;
-            if ((((it >> 1) & 1) ^ turn) && it + 2 < iters) move_sums(it == (SUMS == 1 ? 0 : 2), false);
-        }
-    }
-    if constexpr (SUMS == 1) {
-        if (kw == 0 && iters > 2) move_sums(false, true);
-    } else if constexpr (SUMS == 2) {
-        if (iters > 4) move_sums(false, true);
     }
     // (the loads past the end are not to be dropped: the waits above count them)
 #pragma unroll
@@ -716,7 +655,7 @@ int groups_of(const jl_weight *const *weights, int count) {
 }  // namespace
 
 double jl_gemm_reg_price(const jl_context *ctx, const jl_weight *const *weights, int count, int rows, int epilogue,
-                         bool short_sums, int *tiling) {
+                         int *tiling) {
     *tiling = -1;
     const int type = weights[0]->type, k = (int)weights[0]->cols, column = type_column(type);
     const bool dual = epilogue == JL_SWIGLU;
@@ -730,7 +669,6 @@ double jl_gemm_reg_price(const jl_context *ctx, const jl_weight *const *weights,
     for (int i = 0; i < kTilingCount; i++) {
         const Tiling &t = kTilings[i];
         if (t.full[column] == 0.f) continue;
-        if (short_sums && (k / 256 + t.kw - 1) / t.kw > short_sum_blocks(type, t.mb, t.wn, t.kw)) continue;
         int ntiles, mtiles;
         const int tiles = tiles_of(t, rows, groups, dual, &ntiles, &mtiles);
         const int places = ctx->compute_units * t.places;

@@ -1243,11 +1243,10 @@ static int skinny_window(jl_context *ctx, const jl_weight *const *weights, int c
 }
 
 // Sets *taken to false, launching nothing, when the shape is not one this kernel takes; the caller
-// then uses the tiled GEMM.  `probe`: says in *taken whether it would, and launches nothing.
-// (JL_SKINNY_XH: X16 is read, else X.)
+// then uses the tiled GEMM.  (JL_SKINNY_XH: X16 is read, else X.)
 int JL_SKINNY_ENTRY(jl_context *ctx, const jl_weight *const *weights, int count, const float *X,
                     const _Float16 *X16, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                    int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken, bool probe) {
+                    int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken) {
     // A row is cut into equal spans of whole 256-column blocks, at most eight blocks each, one compute
     // wave per block: a row of 43 blocks (11 008 columns, the feed-forward width of many 7B models) or
     // of 74 (18 944) has no such cut but spans of one or two blocks, on one or two compute waves (100
@@ -1270,10 +1269,6 @@ int JL_SKINNY_ENTRY(jl_context *ctx, const jl_weight *const *weights, int count,
                                plane_bytes, other_us, &tail_ok, head * 4, tail * 4, true);
         if (st != JL_OK) return st;
         if (head_ok && tail_ok) {
-            if (probe) {
-                *taken = true;
-                return JL_OK;
-            }
             st = skinny_window(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue, planes, plane_bytes,
                                other_us, taken, 0, head * 4, false);
             if (st != JL_OK) return st;
@@ -1282,5 +1277,5 @@ int JL_SKINNY_ENTRY(jl_context *ctx, const jl_weight *const *weights, int count,
         }
     }
     return skinny_window(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue, planes, plane_bytes,
-                         other_us, taken, 0, 0, probe);
+                         other_us, taken, 0, 0, false);
 }

@@ -189,25 +189,24 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
 // was one it handles; when not, nothing was launched and the tiled GEMM must run instead.  `X16`
 // set: the activations as binary16 (X is then ignored); `c_f16` (JL_SWIGLU): C holds binary16.
 // `other_us`: what the caller's other way of running a call of 65 .. 511 rows is estimated to take,
-// in microseconds; such a call is taken only when streaming is estimated cheaper.  `probe`: nothing is launched.
+// in microseconds; such a call is taken only when streaming is estimated cheaper.
 int jl_launch_gemm_skinny(jl_context *ctx, const jl_weight *const *weights, int count, const float *X,
                           const _Float16 *X16, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                          int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken, bool probe = false);
+                          int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken);
 // Activation rows one of its workgroups multiplies: 16 or 32; calls of more rows run as two row blocks.
 int jl_skinny_padded_rows(int rows);
 // (its two halves, one translation unit each: fp32 activations, binary16 activations)
 int jl_launch_gemm_skinny_x32(jl_context *ctx, const jl_weight *const *weights, int count, const float *X,
                               const _Float16 *X16, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                              int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken, bool probe);
+                              int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken);
 int jl_launch_gemm_skinny_x16(jl_context *ctx, const jl_weight *const *weights, int count, const float *X,
                               const _Float16 *X16, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                              int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken, bool probe);
+                              int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken);
 // Weights decoded in registers (jl_gemm_reg.hip): what a call with fp32 activations is estimated to take
-// there, in microseconds, and by which tiling; 1e30 when it is not one for that kernel.  `short_sums`: only
-// by a tiling whose fp32 sums are no longer than the weight-streaming kernel's.  The launch reads `rows`
-// rows of A and nothing behind them.
+// there, in microseconds, and by which tiling; 1e30 when it is not one for that kernel.  The launch reads
+// `rows` rows of A and nothing behind them.
 double jl_gemm_reg_price(const jl_context *ctx, const jl_weight *const *weights, int count, int rows, int epilogue,
-                         bool short_sums, int *tiling);
+                         int *tiling);
 int jl_launch_gemm_reg(jl_context *ctx, const jl_weight *const *weights, int count, const _Float16 *A,
                        const float *row_scale, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
                        int epilogue, int tiling);
