@@ -122,7 +122,12 @@ __device__ __forceinline__ float jl_wave_max(float v) {
 // the first value is used, a pass past the row's end re-reads the thread's first columns: under a condition
 // each the loads waited for one another, and without the asm the compiler reads a value again rather
 // than keep it.
-template <int HELD>
+// MARK (rows of whole 256-column blocks): a row with a block that this one scale does not serve has its scale
+// marked by a minus sign.  A wave holds one block in each pass.  Such a block lies more than 2^16 below the
+// row's largest magnitude, and values of it lie below fp16's normal range, where they lose bits or vanish:
+// with block maxima from 2^-16 on, what values lose there is at most 2^-20 of the largest in their block, a two
+// hundredth of what rounding to fp16 takes from that.
+template <int HELD, bool MARK>
 __device__ __forceinline__ void jl_row_to_f16_held(const float *__restrict__ x, _Float16 *__restrict__ a,
                                                    float *__restrict__ row_scale, int k) {
     typedef _Float16 jl_half4 __attribute__((ext_vector_type(4)));
@@ -161,15 +166,38 @@ __device__ __forceinline__ void jl_row_to_f16_held(const float *__restrict__ x, 
     auto put = [&](int i, const jl_float4 &w) {
         *(jl_half4 *)(a + i) = jl_half4{(_Float16)(w[0] * inv), (_Float16)(w[1] * inv), (_Float16)(w[2] * inv), (_Float16)(w[3] * inv)};
     };
+    // (a wave looks at its block's smallest values only where none of the others is large enough)
+    bool mark = false;
+    auto look = [&](const jl_float4 &w) {
+        if (__ballot(largest(w) * inv >= 0x1p-5f) != 0) return;
+        bool under = false;
+#pragma unroll
+        for (int e = 0; e < 4; e++) under = under || (w[e] != 0.f && fabsf(w[e]) * inv < 0x1p-14f);
+        mark = mark || __ballot(under) != 0;
+    };
 #pragma unroll
     for (int j = 0; j < HELD; j++) {
         const int i = tid * 4 + j * 1024;
-        if (i < k) put(i, v[j]);
+        if (i < k) {
+            put(i, v[j]);
+            if constexpr (MARK) look(v[j]);
+        }
     }
-    for (int i = tid * 4 + HELD * 1024; i < k; i += 1024) put(i, *(const jl_float4 *)(x + i));
+    for (int i = tid * 4 + HELD * 1024; i < k; i += 1024) {
+        const jl_float4 w = *(const jl_float4 *)(x + i);
+        put(i, w);
+        if constexpr (MARK) look(w);
+    }
+    if constexpr (MARK) {
+        __shared__ int wave_marks[4];
+        if ((tid & 63) == 0) wave_marks[tid >> 6] = mark;
+        __syncthreads();
+        if (amax < INFINITY && (wave_marks[0] | wave_marks[1] | wave_marks[2] | wave_marks[3])) scale = -scale;
+    }
     if (tid == 0) *row_scale = scale;
 }
 
+template <bool MARK = false>
 __device__ __forceinline__ void jl_row_to_f16(const float *__restrict__ X, _Float16 *__restrict__ A,
                                               float *__restrict__ row_scale, int rows, int k, int row) {
     typedef _Float16 jl_half4 __attribute__((ext_vector_type(4)));
@@ -180,7 +208,7 @@ __device__ __forceinline__ void jl_row_to_f16(const float *__restrict__ X, _Floa
         return;
     }
     const float *x = X + (int64_t)row * k;
-    if (k <= 2048) jl_row_to_f16_held<2>(x, a, row_scale + row, k);
-    else if (k <= 4096) jl_row_to_f16_held<4>(x, a, row_scale + row, k);
-    else jl_row_to_f16_held<8>(x, a, row_scale + row, k);
+    if (k <= 2048) jl_row_to_f16_held<2, MARK>(x, a, row_scale + row, k);
+    else if (k <= 4096) jl_row_to_f16_held<4, MARK>(x, a, row_scale + row, k);
+    else jl_row_to_f16_held<8, MARK>(x, a, row_scale + row, k);
 }

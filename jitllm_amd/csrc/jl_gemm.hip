@@ -39,6 +39,11 @@ jl_rows_to_f16(const float *__restrict__ X, _Float16 *__restrict__ A, float *__r
                int rows, int k) {
     jl_row_to_f16(X, A, row_scale, rows, k, blockIdx.x);
 }
+__global__ void __launch_bounds__(256)
+jl_rows_to_f16_marked(const float *__restrict__ X, _Float16 *__restrict__ A, float *__restrict__ row_scale,
+                      int rows, int k) {
+    jl_row_to_f16<true>(X, A, row_scale, rows, k, blockIdx.x);
+}
 
 // Activations that arrive as fp16 but in a buffer the kernels cannot read whole row tiles of: the
 // active rows copied as they are, the rows that pad the last tile zero-filled.  A thread moves 16 bytes.
@@ -1030,12 +1035,16 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     // activations have.
     const double decoded_us = dense_us + 3.5 + (dsplits > 1 ? 1.5 : 0.0) + (weight_bytes + 2.0 * virt * k) / 4.0e6 + 6.0 * rows * k / 2.9e6;
     if (reg_tiling >= 0 && reg_us < (dense ? decoded_us : in_loop_us)) {
+        // (of Q8_0 and Q4_0 it takes calls from the weight-streaming kernel, which scales every 256 columns of an
+        // activation row by themselves: rows that want that are marked here and done apart there)
+        const bool marks = !X16 && (type == JL_Q8_0 || type == JL_Q4_0);
         if (!X16) {
-            hipLaunchKernelGGL(jl_rows_to_f16, dim3(rows), dim3(256), 0, ctx->stream, X, A, row_scale, rows, k);
+            if (marks) hipLaunchKernelGGL(jl_rows_to_f16_marked, dim3(rows), dim3(256), 0, ctx->stream, X, A, row_scale, rows, k);
+            else hipLaunchKernelGGL(jl_rows_to_f16, dim3(rows), dim3(256), 0, ctx->stream, X, A, row_scale, rows, k);
             JL_HIP(hipGetLastError());
         }
-        return jl_launch_gemm_reg(ctx, weights, count, X16 ? X16 : A, X16 ? nullptr : row_scale, C, c_f16, rows, ldo,
-                                  col_offset, epilogue, reg_tiling);
+        return jl_launch_gemm_reg(ctx, weights, count, X16 ? X16 : A, X16 ? nullptr : row_scale, marks ? X : nullptr, C,
+                                  c_f16, rows, ldo, col_offset, epilogue, reg_tiling);
     }
     // what a kept copy looks like: gate / up interleaved by half tiles of this BN, or plain
     const int32_t layout = epilogue == JL_SWIGLU ? bn : 1;

@@ -62,6 +62,7 @@ struct RegParams {
     const uint8_t *w_up;       // JL_SWIGLU: the up weight
     const _Float16 *A;         // [rows x k]
     const float *row_scale;    // null: every scale is 1
+    const float *X;            // set: rows whose scale is marked by a minus sign are multiplied from here
     float *C;
     int c_f16;                 // JL_SWIGLU: C holds binary16 values, ldo and col_offset count them
     int rows, k;
@@ -207,6 +208,20 @@ __device__ __forceinline__ half8 decode_frag(const HalfWords<TYPE> &s, int t, in
 }
 
 __device__ __forceinline__ float reg_swiglu(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u; }
+
+// One output of a row that no power of two brings into fp16's range block by block: fp32 products of the
+// activations as they came, lanes across the columns.  The sum is in every lane.
+template <int TYPE>
+__device__ __forceinline__ float plain_dot(const uint8_t *w, const float *x, int k, int lane) {
+    float sum = 0.f;
+    for (int c = lane; c < k; c += 64) {
+        const uint8_t *b = w + (c >> 5) * (quad_bytes(TYPE) / 8);
+        const float d = jl_half_bits_to_float(*(const uint16_t *)b);
+        const int q = TYPE == JL_Q8_0 ? (int)(int8_t)b[2 + (c & 31)] : ((b[2 + (c & 15)] >> ((c & 16) >> 2)) & 15) - 8;
+        sum += d * (float)q * x[c];
+    }
+    return jl_group_sum<64>(sum);
+}
 
 // What the chunk position of an activation row is exclusive-ored with.  A 128-bit LDS read serves 16
 // lanes a cycle, rows 0-3 and 12-15 of one slice with rows 4-11 of the next: with slices four chunks
@@ -516,6 +531,7 @@ jl_gemm_reg(RegParams p) {
         const int row = m0 + 16 * m + r16;
         if (row >= p.rows) return;
         const float rs = p.row_scale ? p.row_scale[row] : 1.f;
+        if (rs < 0.f) return;   // (done apart, below)
         const int64_t at = (int64_t)row * p.ldo + p.col_offset + 4 * g;
         if (swiglu) {
             float v[4];
@@ -576,6 +592,35 @@ jl_gemm_reg(RegParams p) {
 #pragma unroll
                 for (int j = 0; j < NR; j++) t[j] += fold[((((z * WN + wn) * MB + m) * NR) + j) * 64 + lane];
             finish(m, t);
+        }
+    }
+    // Rows with a marked scale, which hardly any call has (a wave looks through its tile's scales: 0.1 us)
+    if constexpr (TYPE == JL_Q8_0 || TYPE == JL_Q4_0) {
+        if (!p.X || kw != 0) return;
+        for (int first = 0; first < ROWS; first += 64) {
+            const int mine = first + lane;
+            uint64_t marked = __ballot(mine < ROWS && m0 + mine < p.rows && p.row_scale[m0 + mine] < 0.f);
+            for (; marked; marked &= marked - 1) {
+                const int row = m0 + first + __builtin_ctzll(marked);
+                const float *x = p.X + (int64_t)row * p.k;
+                float *dst = p.C + (int64_t)row * p.ldo + p.col_offset;
+                for (int e = 0; e < kGroup; e++) {
+                    float v[NR];
+#pragma unroll
+                    for (int j = 0; j < NR; j++) v[j] = e < out_from[j] ? 0.f : plain_dot<TYPE>(group_ptr[j] + (int64_t)e * p.row_bytes, x, p.k, lane);
+                    if (lane != 0) continue;
+                    if (swiglu) {
+                        if (e >= out_from[0]) dst[out_col[0] + e] = reg_swiglu(v[0], v[1]);
+                        continue;
+                    }
+#pragma unroll
+                    for (int j = 0; j < NR; j++) {
+                        if (e < out_from[j]) continue;
+                        if (p.epilogue == JL_RESIDUAL) dst[out_col[j] + e] += v[j];
+                        else dst[out_col[j] + e] = v[j];
+                    }
+                }
+            }
         }
     }
 }
@@ -695,8 +740,8 @@ double jl_gemm_reg_price(const jl_context *ctx, const jl_weight *const *weights,
 }
 
 int jl_launch_gemm_reg(jl_context *ctx, const jl_weight *const *weights, int count, const _Float16 *A,
-                       const float *row_scale, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                       int epilogue, int tiling) {
+                       const float *row_scale, const float *X, float *C, bool c_f16, int rows, int64_t ldo,
+                       int64_t col_offset, int epilogue, int tiling) {
     const int type = weights[0]->type, k = (int)weights[0]->cols;
     const bool dual = epilogue == JL_SWIGLU;
     RegParams p{};
@@ -714,6 +759,7 @@ int jl_launch_gemm_reg(jl_context *ctx, const jl_weight *const *weights, int cou
     p.w_up = dual ? weights[1]->blocks : nullptr;
     p.A = A;
     p.row_scale = row_scale;
+    p.X = X;
     p.C = C;
     p.c_f16 = c_f16 ? 1 : 0;
     p.rows = rows;

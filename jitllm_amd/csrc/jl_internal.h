@@ -204,12 +204,13 @@ int jl_launch_gemm_skinny_x16(jl_context *ctx, const jl_weight *const *weights, 
                               int epilogue, float *planes, size_t plane_bytes, double other_us, bool *taken);
 // Weights decoded in registers (jl_gemm_reg.hip): what a call with fp32 activations is estimated to take
 // there, in microseconds, and by which tiling; 1e30 when it is not one for that kernel.  The launch reads
-// `rows` rows of A and nothing behind them.
+// `rows` rows of A and nothing behind them.  `X` set (Q8_0, Q4_0): the fp32 activations, of which rows with a
+// marked scale (jl_row_to_f16) are multiplied as they are.
 double jl_gemm_reg_price(const jl_context *ctx, const jl_weight *const *weights, int count, int rows, int epilogue,
                          int *tiling);
 int jl_launch_gemm_reg(jl_context *ctx, const jl_weight *const *weights, int count, const _Float16 *A,
-                       const float *row_scale, float *C, bool c_f16, int rows, int64_t ldo, int64_t col_offset,
-                       int epilogue, int tiling);
+                       const float *row_scale, const float *X, float *C, bool c_f16, int rows, int64_t ldo,
+                       int64_t col_offset, int epilogue, int tiling);
 // Many-row prefill: weights decoded to fp16 once per call into `copy`, then a plain fp16 GEMM.
 int jl_dense_column_tile(int rows, int k, int out_cols_virtual, int epilogue, int compute_units, int *splits,
                          int *row_tile, int min_rows = 512, bool may_cut_k = true, double *us = nullptr);

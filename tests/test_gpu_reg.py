@@ -141,6 +141,55 @@ def test_output_columns_off_the_vector_width(ctx):
     w.free()
 
 
+# (type, weight rows side by side, activation rows, gate/up, residual): the tilings with one and with two sets of waves
+@pytest.mark.parametrize("t,ds,rows,dual,residual", [
+    (O.Q8_0, (3003, 3003), 257, True, False), (O.Q8_0, (14003,), 449, False, False),
+    (O.Q4_0, (5005,), 300, False, True), (O.Q4_0, (10001, 17), 129, False, False)])
+def test_rows_whose_blocks_lie_far_apart(ctx, t, ds, rows, dual, residual):
+    """fp32 rows whose 256-column blocks differ by 2^30, under weights that are zero where the row is large: a
+    single power of two for the row would leave nothing of the block that counts."""
+    from jitllm_amd import _lib as L, synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("decode in registers, blocks far apart", t, ds, rows, dual, residual)
+    n, block = 512, 34 if t == O.Q8_0 else 18
+    raws = [np.array(synthetic.weight(t, d, n, seed=7140 + i)).reshape(d, n // 32, block) for i, d in enumerate(ds)]
+    for raw in raws:
+        raw[:, :8, :2] = 0                                     # the scales of the first 256 columns
+    raws = [raw.reshape(-1) for raw in raws]
+    X = synthetic.activations((rows, n), seed=7150)
+    X[1::3, :256] *= np.float32(2.0 ** 30)
+    X[2::6, 256:] = 0
+    ws = [ctx.load_weight(t, raw, d, n) for raw, d in zip(raws, ds)]
+    width = ds[0] if dual else sum(ds)
+    base = synthetic.activations((rows, width), seed=7151) if residual else np.full((rows, width), UNTOUCHED, np.float32)
+    proj = QuantizedBatchProjections(ctx, rows, n, sum(ds))
+    outs = []
+    for _ in range(2):
+        out = ctx.from_numpy(base.reshape(-1).copy())
+        proj._gemm(ws, ctx.from_numpy(X), out, rows, width, 0, L.JL_SWIGLU if dual else L.JL_RESIDUAL if residual else L.JL_STORE)
+        ctx.sync()
+        outs.append(out.get().reshape(rows, width))
+    assert np.array_equal(outs[0].view(np.uint32), outs[1].view(np.uint32))
+    X[:, :256] = 0                                             # (what those columns add)
+    at = 0
+    if dual:
+        cols = columns(width)
+        g, u = (O.matmul_batch(t, rows_of(raw, width, cols), X, len(cols), n).astype(np.float64) for raw in raws)
+        mg, mu = (magnitude(t, rows_of(raw, width, cols), X, len(cols), n) for raw in raws)
+        sig = 1.0 / (1.0 + np.exp(-g))
+        bound = F16_BOUND * (1.1 * mg * np.abs(u) + np.abs(g) * sig * mu + 1.1 * F16_BOUND * mg * mu) + 1e-5
+        assert np.all(np.abs(outs[0][:, cols] - g * sig * u) <= bound)
+        return
+    for raw, d in zip(raws, ds):
+        cols = columns(d)
+        part = rows_of(raw, d, cols)
+        old = base[:, at + cols].astype(np.float64) if residual else 0.0
+        # (an fp32 sum with what was there is rounded once: half a unit in the last place of the result)
+        bound = F16_BOUND * magnitude(t, part, X, len(cols), n) + 2.0 ** -24 * np.abs(outs[0][:, at + cols])
+        assert np.all(np.abs(outs[0][:, at + cols] - old - O.matmul_batch(t, part, X, len(cols), n)) <= bound)
+        at += d
+
+
 # columns, weight rows, activation rows of Q6_K calls that the weight-streaming kernel has, whatever the others cost
 @pytest.mark.parametrize("n,d,rows", [(4096, 4096, 384), (8192, 4096, 511), (14336, 4096, 256), (4096, 12288, 408)])
 def test_q6_k_sums_are_as_exact_as_the_streaming_kernels(ctx, n, d, rows):
