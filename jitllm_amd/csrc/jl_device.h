@@ -86,6 +86,13 @@ __device__ __forceinline__ float jl_swiglu_value(float g, float u) {
     return jl_mul_rn(__fdiv_rn(g, denom), u);
 }
 
+// SiLU(g) * u in single precision: g / (1 + exp(-g)) with expf, a few ulp from the host's double
+// form and three orders of magnitude inside the fp16 path's tolerance; the double-precision exp
+// costs about 150 instructions per output, which matters at T x hidden outputs per call.
+__device__ __forceinline__ float jl_swiglu_single(float g, float u) {
+    return g / (1.0f + __expf(-g)) * u;
+}
+
 // Four consecutive results of an output row stored as binary16 (round to nearest even): one
 // 8-byte store when all four lie inside the row and the address allows it.
 __device__ __forceinline__ void jl_store4_f16(_Float16 *dst, const float (&v)[4], int valid) {

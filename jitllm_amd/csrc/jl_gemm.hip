@@ -279,13 +279,6 @@ __device__ __forceinline__ void decode_half_slice(uint32_t raw_row, uint32_t hdr
         for (int j = 0; j < 8; j++) out[i][j] = w[8 * i + j];
 }
 
-// SiLU(g) * u in single precision: g / (1 + exp(-g)) with expf, a few ulp from the host's double
-// form and three orders of magnitude inside the fp16 path's tolerance; the double-precision exp
-// costs about 150 instructions per output, which matters at T x hidden outputs per call.
-__device__ __forceinline__ float gemm_swiglu(float g, float u) {
-    return g / (1.0f + __expf(-g)) * u;
-}
-
 struct GemmParams {
     const uint8_t *w[kMaxWeights];
     int w_begin[kMaxWeights + 1];  // first virtual output column of each weight
@@ -663,7 +656,7 @@ jl_gemm_f16(GemmParams p) {
                     const int col = n0 + wn * (TN / 2) + j * 16 + (lane >> 4) * 4;
                     float v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = gemm_swiglu(acc[i][j][e] * rs, acc[i][j + NB / 2][e] * rs);
+                    for (int e = 0; e < 4; e++) v[e] = jl_swiglu_single(acc[i][j][e] * rs, acc[i][j + NB / 2][e] * rs);
                     if (p.c_f16) {
                         jl_store4_f16((_Float16 *)p.C + (int64_t)m * p.ldo + p.col_offset + col, v, p.n_total - col);
                         continue;
@@ -728,10 +721,10 @@ jl_gemm_reduce(const float *__restrict__ partial, const float *__restrict__ row_
             sg.x += a.x; sg.y += a.y; sg.z += a.z; sg.w += a.w;
             su.x += b.x; su.y += b.y; su.z += b.z; su.w += b.w;
         }
-        v[0] = gemm_swiglu(sg.x * rs, su.x * rs);
-        v[1] = gemm_swiglu(sg.y * rs, su.y * rs);
-        v[2] = gemm_swiglu(sg.z * rs, su.z * rs);
-        v[3] = gemm_swiglu(sg.w * rs, su.w * rs);
+        v[0] = jl_swiglu_single(sg.x * rs, su.x * rs);
+        v[1] = jl_swiglu_single(sg.y * rs, su.y * rs);
+        v[2] = jl_swiglu_single(sg.z * rs, su.z * rs);
+        v[3] = jl_swiglu_single(sg.w * rs, su.w * rs);
         if (c_f16) {
             jl_store4_f16((_Float16 *)C + (int64_t)m * ldo + col_offset + col, v, n_total - col);
             return;

@@ -207,8 +207,6 @@ __device__ __forceinline__ half8 decode_frag(const HalfWords<TYPE> &s, int t, in
     }
 }
 
-__device__ __forceinline__ float reg_swiglu(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u; }
-
 // One output of a row that no power of two brings into fp16's range block by block: fp32 products of the
 // activations as they came, lanes across the columns.  The sum is in every lane.
 template <int TYPE>
@@ -536,7 +534,7 @@ jl_gemm_reg(RegParams p) {
         if (swiglu) {
             float v[4];
 #pragma unroll
-            for (int e = 0; e < 4; e++) v[e] = reg_swiglu(t[0][e] * rs, t[1][e] * rs);
+            for (int e = 0; e < 4; e++) v[e] = jl_swiglu_single(t[0][e] * rs, t[1][e] * rs);
             const int64_t to = at + out_col[0];
             if (p.c_f16 && out_from[0] == 0) {
                 jl_store4_f16((_Float16 *)p.C + to, v, 4);
@@ -610,7 +608,7 @@ jl_gemm_reg(RegParams p) {
                     for (int j = 0; j < NR; j++) v[j] = e < out_from[j] ? 0.f : plain_dot<TYPE>(group_ptr[j] + (int64_t)e * p.row_bytes, x, p.k, lane);
                     if (lane != 0) continue;
                     if (swiglu) {
-                        if (e >= out_from[0]) dst[out_col[0] + e] = reg_swiglu(v[0], v[1]);
+                        if (e >= out_from[0]) dst[out_col[0] + e] = jl_swiglu_single(v[0], v[1]);
                         continue;
                     }
 #pragma unroll

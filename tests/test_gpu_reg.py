@@ -141,6 +141,31 @@ def test_output_columns_off_the_vector_width(ctx):
     w.free()
 
 
+@pytest.mark.parametrize("t", [O.Q4_0, O.Q4_K])
+def test_swiglu_of_exact_sums_has_the_bits_of_the_kernel_that_decodes_in_its_loop(ctx, t):
+    """One activation a row: a sum is one product, exact in any order, and gate/up's results differ by their SiLU
+    alone.  A context that does not cut K runs the call on the kernel that had it before."""
+    from jitllm_amd import _lib as L, synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    from jitllm_amd.runtime import Context
+    n, d, rows = 1792, 12001, 201
+    say("decode in registers, swiglu", t)
+    raws = [synthetic.weight(t, d, n, seed=7160 + i) for i in range(2)]
+    X = np.zeros((rows, n), np.float16)
+    X[np.arange(rows), (np.arange(rows) * 89) % n] = np.linspace(-400, 400, rows)
+    got = []
+    for split_k in (True, False):
+        with Context(0) as c:
+            c.set_split_k(split_k)
+            ws = [c.load_weight(t, raw, d, n) for raw in raws]
+            proj = QuantizedBatchProjections(c, rows, n, 2 * d)
+            out = c.float_array(rows * d)
+            proj._gemm(ws, c.half_from_numpy(X), out, rows, d, 0, L.JL_SWIGLU)
+            c.sync()
+            got.append(out.get())
+    assert np.any(got[0]) and np.array_equal(got[0].view(np.uint32), got[1].view(np.uint32))
+
+
 # (type, weight rows side by side, activation rows, gate/up, residual): the tilings with one and with two sets of waves
 @pytest.mark.parametrize("t,ds,rows,dual,residual", [
     (O.Q8_0, (3003, 3003), 257, True, False), (O.Q8_0, (14003,), 449, False, False),
