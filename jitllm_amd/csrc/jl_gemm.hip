@@ -983,15 +983,39 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     double reg_us = 1e30;
     if (rows < 512 && rows >= (dense_only ? 128 : 65) && !(kept && (rows >= 128 || dense_only)) && workspace_bytes >= head)
         reg_us = jl_gemm_reg_price(ctx, weights, count, rows, epilogue, &reg_tiling);
+    if (reg_tiling >= 0 && !dense_only) {
+        // Against decoding in the loop the fit above is too high for calls whose 128 x 128 tiles come in one or
+        // two rounds over the chip (7 us and 10.8, 13.5 and 12.5 ns a column and round with Q4_0, Q8_0 and Q4_K: Q4_0
+        // gate/up 2 x [12288 x 4096] at 128 rows 50 us, by the fit 59, in registers 60) and, by 7 % and more,
+        // for narrow Q4_0 calls, which cut K.
+        double loop_us = in_loop_us;
+        const int tiles = (virt + 127) / 128 * ((rows + 127) / 128);
+        if (2 * tiles >= ctx->compute_units) {
+            const int rounds = (tiles + ctx->compute_units - 1) / ctx->compute_units;
+            const double whole_us = 7.0 + (type == JL_Q8_0 ? 0.0135 : type == JL_Q4_0 ? 0.0108 : 0.0125) * k * rounds;
+            if (whole_us < loop_us) loop_us = whole_us;
+        } else if (type == JL_Q4_0) {
+            loop_us *= 0.93;
+        }
+        if (reg_us >= loop_us) {
+            reg_us = 1e30;
+            reg_tiling = -1;
+        }
+    }
     if (rows < 512) {
         // batched decode of up to 64 rows, and calls of up to 511 where it is the cheapest: the
         // weight-streaming kernel reads X itself, fp32 or fp16
         bool taken = false;
         double other_us = in_loop_us < copy_us ? in_loop_us : copy_us;
-        // (near equal prices the streaming kernel is the faster one, by up to 8 %, measured)
-        if (1.1 * reg_us < other_us && type != JL_Q4_K && type != JL_Q6_K) other_us = 1.1 * reg_us;
+        // (Near equal prices the streaming kernel is the faster one, by up to 8 %, and plain and residual calls over rows
+        // of whole 2048-column spans take it 3 - 6 us less than its own price: Q4_0 2048 x 2048 at 234 rows over
+        // fp32 activations 11.1 us, by its price 15.2, in registers 13.5.  Over fp16 ones, whose calls go the same
+        // way so as to give the same bits, that takes back up to 15 %.)
+        const double reg_at_least = 1.1 * reg_us + (epilogue != JL_SWIGLU && k % 2048 == 0 ? 3.0 : 0.0);
+        if (reg_at_least < other_us && type != JL_Q4_K && type != JL_Q6_K) other_us = reg_at_least;
         int st = jl_launch_gemm_skinny(ctx, weights, count, X, X16, C, c_f16, rows, ldo, col_offset, epilogue,
                                        planes, plane_bytes, other_us, &taken);
+        if (taken) ctx->last_gemm.store(JL_GEMM_STREAMED, std::memory_order_relaxed);
         if (st != JL_OK || taken) return st;
     }
 
@@ -1025,9 +1049,12 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
     // The decoded copy's way (Q6_K) in microseconds: the GEMM, a launch that decodes the weights at 4.0 TB/s
     // and converts the activations at 2.9, and 1.5 us between launches, all measured.  Both prices are those
     // of fp32 activations whatever came: a call's sums do not depend on which of the two forms its
-    // activations have.
+    // activations have.  From 129 rows on, and more from 257, the copy's way takes less than its price and the
+    // register kernel more (3584 x 3584 + 2 x [512 x 3584] at 511 rows 48 and 73 us, by the prices 66 and 62).
     const double decoded_us = dense_us + 3.5 + (dsplits > 1 ? 1.5 : 0.0) + (weight_bytes + 2.0 * virt * k) / 4.0e6 + 6.0 * rows * k / 2.9e6;
-    if (reg_tiling >= 0 && reg_us < (dense ? decoded_us : in_loop_us)) {
+    const double against = rows > 256 ? 1.25 : rows > 128 ? 1.2 : 1.0;
+    if (reg_tiling >= 0 && (!dense || against * reg_us < decoded_us)) {
+        ctx->last_gemm.store(JL_GEMM_IN_REGISTERS + reg_tiling, std::memory_order_relaxed);
         // (of Q8_0 and Q4_0 it takes calls from the weight-streaming kernel, which scales every 256 columns of an
         // activation row by themselves: rows that want that are marked here and done apart there)
         const bool marks = !X16 && (type == JL_Q8_0 || type == JL_Q4_0);
@@ -1061,6 +1088,7 @@ int jl_launch_gemm(jl_context *ctx, const jl_weight *const *weights, int count, 
             JL_HIP(hipGetLastError());
         }
     }
+    ctx->last_gemm.store(dense ? JL_GEMM_DECODED : JL_GEMM_IN_LOOP, std::memory_order_relaxed);
     if (dense) {
         const int st = jl_launch_gemm_dense(ctx, weights, count, A, row_scale, C, rows, ldo, col_offset, epilogue,
                                             kept ? (_Float16 *)resident->copy : (_Float16 *)planes, decode, bm, bn,

@@ -28,7 +28,14 @@ struct jl_context {
     // false: no GEMM of this context cuts K across work items (jl_context_set_split_k), so that a
     // row's sums are added in one order whatever the call's row count
     bool split_k = true;
+    // the kernel of the last batched projection, one of JL_GEMM_*, for the tests (jl_context_last_gemm)
+    std::atomic<int> last_gemm{0};
 };
+#define JL_GEMM_STREAMED 1          // jl_gemm_skinny
+#define JL_GEMM_IN_LOOP 2           // jl_gemm_f16
+#define JL_GEMM_DECODED 3           // jl_gemm_hh
+#define JL_GEMM_IN_REGISTERS 100    // jl_gemm_reg: this and the number of its tiling
+extern "C" int jl_context_last_gemm(const jl_context *ctx);
 #define JL_CONTEXT_SCRATCH_BYTES 8192
 #define JL_CONTEXT_ARRIVALS 1024
 #define JL_BOUNCE_HALF_BYTES (8u << 20)

@@ -14,6 +14,14 @@ def say(*parts) -> None:
     print("[gpu-case]", *parts, flush=True)
 
 
+# what a context's last batched projection ran (jl_context_last_gemm); IN_REGISTERS + the number of its tiling
+STREAMED, IN_LOOP, DECODED, IN_REGISTERS = 1, 2, 3, 100
+
+
+def last_gemm(ctx) -> int:
+    return ctx._lib.jl_context_last_gemm(ctx.handle)
+
+
 def magnitude(t: int, raw: np.ndarray, X: np.ndarray, d: int, n: int) -> np.ndarray:
     """sum_j |w_ij x_bj| in float64, [B x d] (or [d] for a vector)."""
     w = np.abs(NP.DEQUANT[t](raw).reshape(d, n).astype(np.float64))

@@ -5,7 +5,7 @@ from __future__ import annotations
 import numpy as np
 import pytest
 
-from gpu_util import magnitude, rel_err, say
+from gpu_util import DECODED, IN_LOOP, IN_REGISTERS, STREAMED, last_gemm, magnitude, rel_err, say
 from oracle import pyoracle as O
 
 pytestmark = pytest.mark.gpu
@@ -139,6 +139,36 @@ def test_output_columns_off_the_vector_width(ctx):
     assert rel_err(got, O.matmul_batch(t, raw, Y, d, n), magnitude(t, raw, Y, d, n)) < F16_BOUND
     proj.workspace.free()
     w.free()
+
+
+# (type, columns, weight rows, activation rows, gate/up or residual, kernel): what measuring both kernels showed to be the faster
+@pytest.mark.parametrize("t,n,ds,rows,epilogue,kernel", [
+    (O.Q4_0, 4096, (12288, 12288), 128, "dual", IN_LOOP), (O.Q8_0, 2048, (8192, 8192), 161, "dual", IN_LOOP),
+    (O.Q4_0, 12288, (4096,), 224, "residual", IN_LOOP), (O.Q4_0, 2048, (2048,), 234, "residual", STREAMED),
+    (O.Q4_0, 4096, (4096,), 289, "residual", STREAMED), (O.Q8_0, 2048, (2048, 512, 512), 257, "", STREAMED),
+    (O.Q6_K, 3584, (3584, 512, 512), 511, "", DECODED), (O.Q6_K, 13824, (5120,), 511, "residual", DECODED),
+    (O.Q6_K, 4096, (14336, 14336), 480, "dual", STREAMED),
+    (O.Q4_0, 4096, (12288, 12288), 161, "dual", IN_REGISTERS), (O.Q8_0, 4096, (11008, 11008), 129, "dual", IN_REGISTERS),
+    (O.Q4_K, 4096, (11008, 11008), 201, "dual", IN_REGISTERS), (O.Q6_K, 11008, (4096,), 201, "residual", IN_REGISTERS)])
+def test_calls_go_to_the_faster_kernel(ctx, t, n, ds, rows, epilogue, kernel):
+    """Both forms of activations the same way: the results have the same bits."""
+    from jitllm_amd import _lib as L
+    from jitllm_amd.ggml import GGMLType
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("which kernel", t, n, ds, rows, epilogue)
+    ws = [ctx.load_weight(t, np.zeros(GGMLType(t).byte_size_for(d * n), np.uint8), d, n) for d in ds]
+    dual = epilogue == "dual"
+    width = ds[0] if dual else sum(ds)
+    proj = QuantizedBatchProjections(ctx, rows, n, sum(ds))
+    out = ctx.float_array(rows * width)
+    for x in (ctx.float_array(rows * n), ctx.half_from_numpy(np.zeros((rows, n), np.float16))):
+        proj._gemm(ws, x, out, rows, width, 0, L.JL_SWIGLU if dual else L.JL_RESIDUAL if epilogue else L.JL_STORE)
+        ctx.sync()
+        ran = last_gemm(ctx)
+        assert (ran if ran < IN_REGISTERS else IN_REGISTERS) == kernel
+    proj.workspace.free()
+    for w in ws:
+        w.free()
 
 
 @pytest.mark.parametrize("t", [O.Q4_0, O.Q4_K])
