@@ -439,7 +439,8 @@ def test_rows_cut_across_workgroups_are_folded_afresh_on_every_call(ctx, t, d, n
 # (type, weight rows, row length, batch, active rows, residual): 65 .. 511 rows on the
 # weight-streaming kernel as 3 .. 16 row blocks -- a last block of one row, partial batches, rows cut
 # across workgroups (more than 2048 columns) with up to eight blocks' partial sums in the workspace,
-# the types whose other way decodes the whole weight first
+# the types whose other way decodes the whole weight first (Q4_0 2048 x 256, sixteen blocks when it came, is
+# decoded in registers now; Q5_K and IQ4_XS have no such kernel)
 MID_ROWS = [
     (O.Q8_0, 520, 2048, 65, 65, False),
     (O.Q8_0, 520, 2048, 160, 131, True),
@@ -450,6 +451,8 @@ MID_ROWS = [
     (O.Q6_K, 300, 2048, 200, 170, False),
     (O.Q5_K, 520, 4096, 384, 384, True),
     (O.IQ4_XS, 264, 1024, 97, 97, False),
+    (O.Q5_K, 264, 4096, 511, 490, True),
+    (O.IQ4_XS, 264, 2048, 511, 511, False),
 ]
 
 

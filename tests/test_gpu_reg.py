@@ -34,9 +34,8 @@ def rows_of(raw, d, cols):
     return np.ascontiguousarray(raw.reshape(d, -1)[cols]).reshape(-1)
 
 
-# (type, columns, weight rows side by side, activation rows, active, gate/up, residual): every tiling of
-# every type, as the kernel's price list chooses them (a kernel trace of this file shows each instance);
-# one block of columns (a set of waves idle), odd block counts, rows of one group, weights whose last group
+# (type, columns, weight rows side by side, activation rows, active, gate/up, residual), wherever the prices send
+# them: one block of columns (a set of waves idle), odd block counts, rows of one group, weights whose last group
 # overlaps the one before
 CASES = [
     (O.Q4_0, 512, (14003,), 449, 449, False, False), (O.Q4_0, 256, (14003, 14003), 200, 200, True, False),
@@ -62,8 +61,42 @@ CASES = [
 ]
 
 
+# (tiling, type, columns, weight rows side by side, activation rows, gate/up, residual): every instance of the kernel,
+# the shape chosen for it by the price list, with four blocks of columns and more to a set of waves -- each block's
+# bytes come in two blocks before they are multiplied -- and an odd count, whose last block one of two sets does not have
+TILINGS = [
+    (0, O.Q8_0, 1280, (14003,), 449, False, False), (1, O.Q8_0, 1280, (12001,), 481, False, True),
+    (2, O.Q8_0, 1280, (10001,), 481, False, False), (3, O.Q8_0, 1280, (4099, 4099), 385, True, False),
+    (6, O.Q8_0, 1792, (5005,), 385, False, False), (7, O.Q8_0, 8448, (2050, 2050), 353, True, False),
+    (8, O.Q8_0, 1280, (4099,), 385, False, False), (9, O.Q8_0, 2816, (1002, 1002), 353, True, False),
+    (10, O.Q8_0, 4352, (1002, 1002), 225, True, False), (0, O.Q4_0, 1280, (14003,), 449, False, False),
+    (1, O.Q4_0, 1280, (12001,), 481, False, True), (2, O.Q4_0, 1280, (10001,), 481, False, False),
+    (3, O.Q4_0, 1280, (4099, 4099), 385, True, False), (4, O.Q4_0, 1792, (3003, 3003), 481, True, False),
+    (5, O.Q4_0, 1792, (5005,), 481, False, True), (6, O.Q4_0, 1792, (4099,), 449, False, False),
+    (7, O.Q4_0, 1792, (4099,), 353, False, True), (8, O.Q4_0, 1280, (4099,), 385, False, False),
+    (9, O.Q4_0, 1792, (1002, 1002), 385, True, False), (10, O.Q4_0, 2816, (600, 600), 353, True, False),
+    (0, O.Q4_K, 1280, (14003,), 449, False, False), (1, O.Q4_K, 1280, (12001,), 481, False, True),
+    (2, O.Q4_K, 1280, (10001,), 481, False, False), (3, O.Q4_K, 1280, (10001,), 385, False, True),
+    (4, O.Q4_K, 2304, (3003, 3003), 481, True, False), (5, O.Q4_K, 2304, (3003, 3003), 449, True, False),
+    (6, O.Q4_K, 2816, (2050, 2050), 449, True, False), (7, O.Q4_K, 2816, (2050, 2050), 353, True, False),
+    (8, O.Q4_K, 2816, (5005, 5005), 161, True, False), (9, O.Q4_K, 2816, (1002, 1002), 385, True, False),
+    (7, O.Q6_K, 5888, (2050, 2050), 225, True, False), (8, O.Q6_K, 1792, (4099,), 385, False, False),
+    (9, O.Q6_K, 1792, (600, 600), 417, True, False), (10, O.Q6_K, 1792, (33,), 129, False, False),
+]
+
+
 @pytest.mark.parametrize("t,n,ds,rows,active,dual,residual", CASES)
 def test_weights_decoded_in_registers(ctx, t, n, ds, rows, active, dual, residual):
+    check(ctx, t, n, ds, rows, active, dual, residual)
+
+
+@pytest.mark.parametrize("tiling,t,n,ds,rows,dual,residual", TILINGS)
+def test_every_tiling_beyond_its_first_blocks(ctx, tiling, t, n, ds, rows, dual, residual):
+    check(ctx, t, n, ds, rows, rows, dual, residual)
+    assert last_gemm(ctx) == IN_REGISTERS + tiling
+
+
+def check(ctx, t, n, ds, rows, active, dual, residual):
     """Against the oracle for fp32 activations; binary16 ones of the same values give the same bits, a
     second call gives the same bits as the first, rows past the active ones stay as they were."""
     from jitllm_amd import _lib as L, synthetic
