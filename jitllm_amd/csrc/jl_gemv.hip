@@ -1481,8 +1481,41 @@ int launch_tiles(jl_context *ctx, const GemvParams &p, int threads, int lds, boo
     return launch_tiles_of<TYPE, DUAL, false>(ctx, p, threads, lds);
 }
 
-// the argmax form of a projection, below
-int launch_argmax_of(jl_context *ctx, const GemvParams &p, int type, int threads, int lds, bool fixed, int *cells);
+// The argmax form of a plain or RMS-folding projection with rows padded to SP slices.
+template <int TYPE, int SP>
+int launch_argmax_sp(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
+    if (p.S == p.Sp) {
+        return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells)
+                       : launch_tiles_of<TYPE, false, false, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells);
+    }
+    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells)
+                   : launch_tiles_of<TYPE, false, false, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells);
+}
+// One main-type weight, whole tiles of in-wave rows (513 ... 4096 columns), stored (not accumulated) outputs.
+// Elsewhere the logits are scanned in a launch of their own: 151936 x 896 Q8_0 with its argmax, call after call, 31.1 us
+// with the scan, 30.9 with cells, 29.9 with cells that the fold reads in one trip.  Q6_K on its fixed-geometry
+// instances gained nothing (a token with a 152064 x 3584 vocabulary 1503 and 1504 us).
+template <int TYPE>
+int launch_argmax(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed, int *cells) {
+    if (fixed && threads == 256) {
+        switch (p.Sp) {
+            case 16: return launch_argmax_sp<TYPE, 16>(ctx, p, lds, cells);
+            case 32: return launch_argmax_sp<TYPE, 32>(ctx, p, lds, cells);
+            case 64: return launch_argmax_sp<TYPE, 64>(ctx, p, lds, cells);
+            default: break;
+        }
+    }
+    return JL_NO_CELLS_FORM;
+}
+
+int launch_argmax_of(jl_context *ctx, const GemvParams &p, int type, int threads, int lds, bool fixed, int *cells) {
+    switch (type) {
+        case JL_Q8_0: return launch_argmax<JL_Q8_0>(ctx, p, threads, lds, fixed, cells);
+        case JL_Q4_0: return launch_argmax<JL_Q4_0>(ctx, p, threads, lds, fixed, cells);
+        case JL_Q4_K: return launch_argmax<JL_Q4_K>(ctx, p, threads, lds, fixed, cells);
+        default: return JL_NO_CELLS_FORM;
+    }
+}
 
 template <int TYPE>
 int launch_generic(jl_context *ctx, const jl_weight *w, const jl_weight *w_up, const float *x,
@@ -1699,43 +1732,3 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
                            "no single-token projection kernel for a ggml type %d weight", type);
     }
 }
-
-namespace {
-
-// The argmax form of a plain or RMS-folding projection with rows padded to SP slices.
-template <int TYPE, int SP>
-int launch_argmax_sp(jl_context *ctx, const GemvParams &p, int lds, int *cells) {
-    if (p.S == p.Sp) {
-        return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells)
-                       : launch_tiles_of<TYPE, false, false, false, 256, SP, false, false, true>(ctx, p, 256, lds, cells);
-    }
-    return p.rms_w ? launch_tiles_of<TYPE, false, true, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells)
-                   : launch_tiles_of<TYPE, false, false, false, 256, SP, false, true, true>(ctx, p, 256, lds, cells);
-}
-// One main-type weight, whole tiles of in-wave rows (513 ... 4096 columns), stored (not accumulated) outputs.
-// Elsewhere the logits are scanned in a launch of their own: 151936 x 896 Q8_0 with its argmax 35.1 us with the
-// scan, 31.8 with cells (a token of that model 435 -> 426 us).  Q6_K on its fixed-geometry instances gained
-// nothing (a token with a 152064 x 3584 vocabulary 1503 and 1504 us).
-template <int TYPE>
-int launch_argmax(jl_context *ctx, const GemvParams &p, int threads, int lds, bool fixed, int *cells) {
-    if (fixed && threads == 256) {
-        switch (p.Sp) {
-            case 16: return launch_argmax_sp<TYPE, 16>(ctx, p, lds, cells);
-            case 32: return launch_argmax_sp<TYPE, 32>(ctx, p, lds, cells);
-            case 64: return launch_argmax_sp<TYPE, 64>(ctx, p, lds, cells);
-            default: break;
-        }
-    }
-    return JL_NO_CELLS_FORM;
-}
-
-int launch_argmax_of(jl_context *ctx, const GemvParams &p, int type, int threads, int lds, bool fixed, int *cells) {
-    switch (type) {
-        case JL_Q8_0: return launch_argmax<JL_Q8_0>(ctx, p, threads, lds, fixed, cells);
-        case JL_Q4_0: return launch_argmax<JL_Q4_0>(ctx, p, threads, lds, fixed, cells);
-        case JL_Q4_K: return launch_argmax<JL_Q4_K>(ctx, p, threads, lds, fixed, cells);
-        default: return JL_NO_CELLS_FORM;
-    }
-}
-
-}  // namespace
