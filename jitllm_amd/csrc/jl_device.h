@@ -92,6 +92,8 @@ __device__ __forceinline__ float jl_swiglu_value(float g, float u) {
 __device__ __forceinline__ float jl_swiglu_single(float g, float u) {
     return g / (1.0f + __expf(-g)) * u;
 }
+// ... with the reciprocal instruction, up to a unit in the last place from the quotient
+__device__ __forceinline__ float jl_swiglu_rcp(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u; }
 
 // Four consecutive results of an output row stored as binary16 (round to nearest even): one
 // 8-byte store when all four lie inside the row and the address allows it.

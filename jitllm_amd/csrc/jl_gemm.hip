@@ -21,10 +21,10 @@
 
 #include "jl_device.h"
 #include "jl_internal.h"
+#include "jl_slice_decode.h"
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
 typedef _Float16 half4 __attribute__((ext_vector_type(4)));
 typedef _Float16 half2_t __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
@@ -178,17 +178,8 @@ __device__ __forceinline__ void lds_read_3x4(uint32_t a0, uint32_t a1, uint4 &h,
 
 // ---- weight decode: raw block bytes -> fp16, two elements per instruction ----------------------
 //
-// A byte b in 0..255 placed under the exponent byte 0x64 is the fp16 number 1024 + b, exactly; one
-// packed subtract recentres it (1152 = 1024 + 128 for a sign-flipped int8, 1032 = 1024 + 8 for a
-// nibble), one packed multiply applies the block scale.  Both products are exact before their one
-// rounding, so the result is the host's float decode rounded once to fp16.
-
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
-
-__device__ __forceinline__ h2 bytes_to_h2(uint32_t v, uint32_t sel) {
-    // sel picks two bytes of v (selector values 4..7) and pairs each with 0x64 (selector 0)
-    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(v, 0x64646464u, sel));
-}
+// By bytes_to_h2 (jl_slice_decode.h): one packed subtract recentres a byte (1152 = 1024 + 128 for a
+// sign-flipped int8, 1032 = 1024 + 8 for a nibble), one packed multiply applies the block scale.
 
 // 4 bytes (already in 0..255 "offset" form) -> 4 fp16 = (byte - bias) * d
 __device__ __forceinline__ void dword_to_h4(uint32_t v, h2 bias, h2 d, _Float16 *dst) {

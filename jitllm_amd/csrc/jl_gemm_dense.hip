@@ -14,11 +14,10 @@
 //                      share of both operands by LDS-DMA, the two waves of a SIMD half a step apart
 #include "jl_device.h"
 #include "jl_internal.h"
+#include "jl_slice_decode.h"
 
 namespace {
 
-typedef _Float16 half8 __attribute__((ext_vector_type(8)));
-typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
@@ -27,10 +26,6 @@ typedef __attribute__((address_space(3))) void lvoid;
     __builtin_amdgcn_s_waitcnt(((N)&0xF) | (((N) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
 
 // ---- weights -> fp16 ---------------------------------------------------------------------------
-
-__device__ __forceinline__ h2 bytes_to_h2(uint32_t v, uint32_t sel) {
-    return __builtin_bit_cast(h2, __builtin_amdgcn_perm(v, 0x64646464u, sel));
-}
 
 // four bytes in 0..255 offset form -> (byte - bias) * d, four fp16
 __device__ __forceinline__ void dword_scaled(uint32_t v, h2 bias, h2 d, h2 &lo, h2 &hi) {
@@ -248,8 +243,6 @@ struct DenseParams {
     int splits;              // K is cut into `splits` equal runs of steps, one work item each
     float *partial;          // splits > 1: [splits][mtiles * BM][ntiles * BN] fp32 partial sums
 };
-
-__device__ __forceinline__ float dense_swiglu(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u; }
 
 constexpr int DBK = 64;
 constexpr int kRowPad = 256;   // activation rows are padded to whole tiles of the largest row tile
@@ -531,7 +524,7 @@ jl_gemm_hh(DenseParams p) {
                     const int col = n0 + wn * (TN / 2) + j * 16 + (lane >> 4) * 4;
                     float v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = dense_swiglu(acc[i][j][e] * rs, acc[i][j + NB / 2][e] * rs);
+                    for (int e = 0; e < 4; e++) v[e] = jl_swiglu_rcp(acc[i][j][e] * rs, acc[i][j + NB / 2][e] * rs);
                     if (p.c_f16) {
                         jl_store4_f16((_Float16 *)p.C + (int64_t)m * p.ldo + p.col_offset + col, v, p.n_total - col);
                         continue;

@@ -480,8 +480,6 @@ __device__ __forceinline__ uint32_t scaled_pair_f16(float a, float b, float scal
     return r;
 }
 
-__device__ __forceinline__ float skinny_swiglu(float g, float u) { return g * __builtin_amdgcn_rcpf(1.0f + __expf(-g)) * u; }
-
 // Workgroup = 16 Ss compute threads (Ss / 4 waves) + kDmaWaves waves that do nothing but copy tiles.
 // An LDS-DMA load holds its wave at issue while the memory system is busy; issued from the compute
 // waves that time adds to the arithmetic instead of hiding behind it, so the copies have waves of
@@ -581,7 +579,7 @@ __global__ void __launch_bounds__(512 + 64 * (kDmaWaves + kFoldWaves)) jl_gemm_s
 #pragma unroll
         for (int e = 0; e < 4; e++) {
             if (m0 + e >= p.rows) break;
-            const float r = DUAL ? skinny_swiglu(sum[e], sum_up[e]) : sum[e];
+            const float r = DUAL ? jl_swiglu_rcp(sum[e], sum_up[e]) : sum[e];
             if (XH && DUAL && p.c_f16) ((_Float16 *)p.C)[at + e * p.ldo] = (_Float16)r;   // rounded once from the fp32 value
             else if (p.epilogue == JL_RESIDUAL) unsafeAtomicAdd(dst + e * p.ldo, r);   // one add per element, no load to wait for
             else dst[e * p.ldo] = r;

@@ -1,5 +1,5 @@
-// Raw quant bytes to fp16 MFMA fragments in registers: the arithmetic that the kernels which decode
-// weights as they stream by have in common (jl_gemm_skinny_kernels.h, jl_gemm_reg.hip).
+// Raw quant bytes to fp16: the arithmetic that the kernels which decode weights have in common
+// (jl_gemm_skinny_kernels.h and jl_gemm_reg.hip; of it jl_gemm.hip and jl_gemm_dense.hip take bytes_to_h2).
 #pragma once
 
 #include "jl_device.h"
@@ -16,6 +16,7 @@ typedef _Float16 h2 __attribute__((ext_vector_type(2)));
 // subtract recentres it and a packed multiply applies the block scale.  Each product is exact
 // before its one rounding, so a decoded weight is the host's float decode rounded once to fp16.
 
+// `sel` picks two bytes of v (selector values 4..7) and pairs each with 0x64 (selector 0).
 __device__ __forceinline__ h2 bytes_to_h2(uint32_t v, uint32_t sel) {
     return __builtin_bit_cast(h2, __builtin_amdgcn_perm(v, 0x64646464u, sel));
 }
