@@ -386,7 +386,8 @@ int jl_gemm(jl_context *ctx, const jl_weight *const *weights, int count, const f
  * jl_weight comes back at the old address.  Calls that do not decode ignore both.  Results are the
  * same as jl_gemm's, bit for bit -- except that calls of 128 .. 511 rows may run the plain fp16 GEMM
  * over a kept copy where jl_gemm, which would have to decode first, runs a kernel that decodes as it
- * goes: the same products of the same fp16 operands, added in fp32 in another order.
+ * goes: products of the same operands, added in fp32 in another order, or (Q6_K, and Q4_K where it
+ * streams its weights) of weights that are not rounded to fp16 first, as those of the copy are.
  */
 size_t jl_gemm_resident_bytes(const jl_weight *const *weights, int count);
 int jl_gemm_resident(jl_context *ctx, const jl_weight *const *weights, int count, const float *X, float *C,

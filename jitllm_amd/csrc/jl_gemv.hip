@@ -1630,9 +1630,12 @@ int jl_launch_gemv(jl_context *ctx, const jl_weight *const *w, int nseg, float *
         // measured: the tile kernel is the faster one from rows of 2048 columns and 2 MB of weights
         // (by up to 1.7 x on the vocabulary and feed-forward projections), and below 2 MB on whole tiles of Q6_K rows that
         // fill their slices, plain and residual: 512 x 4096 4.0 us on the one-wave-per-row kernel and 3.1 here, 256 x 8192
-        // 5.8 and 3.5, 512 x 2048 2.80 and 2.76 (48 x 2048 2.54 and 2.58: of that length from 128 KB on).  On other Q6_K rows it is the faster one too (512 x 3584 4.4 and 3.3),
-        // but up to 2.4 % further from the float64 values (3584 columns, 2-norm: 1.514e-7 and 1.526e-7; whole rows
-        // 4096 columns 1.534e-7 and 1.528e-7): those stay.  Q5_K loses 2 - 4 % at 2304 - 3072 columns.
+        // 5.8 and 3.5, 512 x 2048 2.80 and 2.76 (48 x 2048 2.54 and 2.58: of that length from 128 KB on).  On other Q6_K
+        // rows it is the faster one too (512 x 3584 4.4 and 3.3), but 0.3 - 1.2 % further from the float64 values: 2-norm,
+        // one wave a row and tiles, over a million results each, known to 0.1 %: 2304 columns 1.511e-7 and 1.530e-7, 3584
+        // 1.528e-7 and 1.538e-7, 6144 1.550e-7 and 1.555e-7; rows that fill their slices 2048 columns 1.507e-7 and
+        // 1.501e-7, 4096 1.528e-7 and 1.525e-7, 8192 1.571e-7 and 1.552e-7.  Q5_K loses 2 - 4 % of its time at 2304 - 3072
+        // columns.
         // (Q6_K rows whose tiles start off a 16-byte boundary, every super-block count from 9 to 63 at 2 MB, 1024,
         // 3584, 8192 and 32768 rows: 0.44 - 0.94 of the one-wave-per-row kernel's time, also where half of a tile's
         // threads have no slice -- 17 super-blocks: 592 rows 5.05 and 4.55 us, 8192 rows 16.8 and 12.1 -- and from 61,
