@@ -278,6 +278,28 @@ def test_rows_whose_blocks_lie_far_apart(ctx, t, ds, rows, dual, residual):
         at += d
 
 
+@pytest.mark.parametrize("t,n,d,rows", [(O.Q8_0, 1280, 4099, 385), (O.Q4_0, 1280, 4099, 385), (O.Q4_K, 1280, 10001, 385),
+                                        (O.Q6_K, 1792, 4099, 385)])
+def test_binary16_subnormals_are_multiplied(ctx, t, n, d, rows):
+    """Rows of binary16 subnormals, which no scale brings into the normal range on this kernel."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("decode in registers, subnormals", t, n, d, rows)
+    raw = synthetic.weight(t, d, n, seed=7170)
+    w = ctx.load_weight(t, raw, d, n)
+    X = np.random.default_rng(7171).integers(-1000, 1001, (rows, n)).astype(np.float64) * 2.0 ** -24
+    proj = QuantizedBatchProjections(ctx, rows, n, d)
+    out = ctx.float_array(rows * d)
+    proj.projection(ctx.half_from_numpy(X.astype(np.float16)), out, w, n, d, False)
+    ctx.sync()
+    assert last_gemm(ctx) >= IN_REGISTERS
+    cols = columns(d)
+    part = rows_of(raw, d, cols)
+    x = X.astype(np.float32)
+    assert rel_err(out.get().reshape(rows, d)[:, cols], O.matmul_batch(t, part, x, len(cols), n), magnitude(t, part, x, len(cols), n)) < F16_BOUND
+    w.free()
+
+
 # columns, weight rows, activation rows of Q6_K calls that the weight-streaming kernel has, whatever the others cost
 @pytest.mark.parametrize("n,d,rows", [(4096, 4096, 384), (8192, 4096, 511), (14336, 4096, 256), (4096, 12288, 408)])
 def test_q6_k_sums_are_as_exact_as_the_streaming_kernels(ctx, n, d, rows):
