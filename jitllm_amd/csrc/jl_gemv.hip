@@ -495,25 +495,17 @@ __device__ __forceinline__ float slice_dot_packed_q4_k(const uint4 &h, const uin
 typedef __attribute__((address_space(1))) const void gvoid;
 typedef __attribute__((address_space(3))) void lvoid;
 
+// The bytes of a tile as a buffer: weights are brought in by buffer loads, whose completion the compiler counts
+// exactly.  With a global load to LDS under way -- an instruction of the flat family -- it answers the first use of
+// any other loaded value with a wait for everything: the normalising launches, whose activations are asked for before
+// the first tile, then began their sum of squares when that tile had landed.
+__device__ __forceinline__ __amdgpu_buffer_rsrc_t tile_bytes(const uint8_t *p) {
+    return __builtin_amdgcn_make_buffer_rsrc((void *)p, 0, -1, 0x00020000);
+}
+
 // s_waitcnt vmcnt(N) only (gfx9 encoding: vmcnt in bits 3:0 and 15:14, expcnt 6:4, lgkmcnt 11:8).
 #define JL_WAIT_VM(N) \
     __builtin_amdgcn_s_waitcnt(((N)&0xF) | (((N) >> 4) << 14) | (0x7 << 4) | (0xF << 8))
-
-// Waits until at most `tiles` tiles' worth of loads (PER_TILE each) are outstanding; every case is
-// an immediate, as the instruction requires.
-template <int PER_TILE>
-__device__ __forceinline__ void wait_vm_tiles(int tiles) {
-    switch (tiles) {
-        case 0: JL_WAIT_VM(0); break;
-        case 1: JL_WAIT_VM(PER_TILE); break;
-        case 2: JL_WAIT_VM(2 * PER_TILE); break;
-        case 3: JL_WAIT_VM(3 * PER_TILE); break;
-        case 4: JL_WAIT_VM(4 * PER_TILE); break;
-        case 5: JL_WAIT_VM(5 * PER_TILE); break;
-        case 6: JL_WAIT_VM(6 * PER_TILE); break;
-        default: JL_WAIT_VM(7 * PER_TILE); break;
-    }
-}
 
 // two consecutive dwords from a four-byte aligned address
 __device__ __forceinline__ uint2 lds_read_b64(uint32_t addr) {
@@ -823,19 +815,13 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     const uint32_t ring0 = lds0 + kPartialBytes;
     uint8_t *ring = lds + kPartialBytes;
 
-    // Per-thread byte offsets of its L load slots inside a tile; for a gate/up tile the slots past
-    // half_bytes read the up weight.
-    int slot_off[L];
-    bool slot_up[L];
-#pragma unroll
-    for (int k = 0; k < L; k++) {
-        int off = k < X4 ? (k * nthreads + tid) * 16 : X4 * nthreads * 16 + tid * 4;
-        slot_up[k] = DUAL && off >= half_bytes;
-        slot_off[k] = slot_up[k] ? off - half_bytes : off;
-    }
+    // A gate/up stage is two halves, one weight's rows each: load slots are dealt so that a wave's 64 lanes
+    // always read the same weight, and rows of the up weight lie `up_at` bytes past the gate's first.
+    const int nwaves = nthreads / JL_WAVE;
+    const int up_at = stage_bytes / 2;
 
     // Brings tile `tile` into stage `st`.  Every thread issues exactly L loads, whatever the tile:
-    // lanes that have nothing to fetch re-read the segment's first bytes into their own slot, so
+    // lanes that have nothing to fetch re-read the tile's first bytes into their own slot, so
     // each wave's outstanding-load count is a compile-time constant per tile.
     // (a launch with one segment -- every one but the fused q|k|v -- never indexes the argument
     // arrays with a run-time segment: that is a scalar memory load, and a wait, per tile)
@@ -890,39 +876,41 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         const uint8_t *base_up = DUAL ? w_up_first + offset : base;
         uint8_t *dst = ring + st * stage_bytes;
         const bool whole = exact && (FULL || bytes == half_bytes);  // uniform
-        if (whole) {
+#pragma unroll
+        for (int k = 0; k < L; k++) {
+            const int width = k < X4 ? 16 : 4;
+            // the wave's place among the loads of this width, and where those begin
+            int unit = k < X4 ? k * nwaves + wave : wave;
+            const int units = (k < X4 ? X4 : 1) * nwaves;
+            int begin = k < X4 ? 0 : X4 * nthreads * 16;
+            const bool up = DUAL && unit >= units / 2;
+            if (up) unit -= units / 2;
+            if (DUAL) begin /= 2;
+            const int at = begin + unit * JL_WAVE * width;
+            uint8_t *to = dst + (up ? up_at : 0) + at;
+            const auto from = tile_bytes(up ? base_up : base);
+            // (a shifted tile's last 16 bytes may run past its end, not past the weight's, whose
+            // bytes are a multiple of 16)
+            const int off = at + lane * width;
+            const bool real = whole || (kShiftedTiles ? off < bytes : off + width <= bytes);
             // the usual case (uniform): every slot is inside the tile, nothing to redirect
-#pragma unroll
-            for (int k = 0; k < L; k++) {
-                const int wave_off = k < X4 ? (k * nthreads + wave * JL_WAVE) * 16
-                                            : X4 * nthreads * 16 + wave * JL_WAVE * 4;
-                const uint8_t *src = (DUAL && slot_up[k] ? base_up : base) + slot_off[k];
-                if (k < X4)
-                    __builtin_amdgcn_global_load_lds((gvoid *)src, (lvoid *)(dst + wave_off), 16, 0, DUAL ? kStreamNonTemporal : 0);
-                else
-                    __builtin_amdgcn_global_load_lds((gvoid *)src, (lvoid *)(dst + wave_off), 4, 0, DUAL ? kStreamNonTemporal : 0);
-            }
-        } else {
-#pragma unroll
-            for (int k = 0; k < L; k++) {
-                const int width = k < X4 ? 16 : 4;
-                const int wave_off = k < X4 ? (k * nthreads + wave * JL_WAVE) * 16
-                                            : X4 * nthreads * 16 + wave * JL_WAVE * 4;
-                const uint8_t *src = (DUAL && slot_up[k] ? base_up : base) + slot_off[k];
-                // (a shifted tile's last 16 bytes may run past its end, not past the weight's, whose
-                // bytes are a multiple of 16)
-                if (kShiftedTiles ? slot_off[k] >= bytes : slot_off[k] + width > bytes) src = wseg;
-                if (k < X4)
-                    __builtin_amdgcn_global_load_lds((gvoid *)src, (lvoid *)(dst + wave_off), 16, 0, 0);
-                else
-                    __builtin_amdgcn_global_load_lds((gvoid *)src, (lvoid *)(dst + wave_off), 4, 0, 0);
+            const int lane_off = whole ? lane * width : real ? off : 0, wave_off = whole ? at : 0;
+            if (k < X4) {
+                if (DUAL && whole) __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lvoid *)to, 16, lane_off, wave_off, 0, kStreamNonTemporal);
+                else __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lvoid *)to, 16, lane_off, wave_off, 0, 0);
+            } else {
+                if (DUAL && whole) __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lvoid *)to, 4, lane_off, wave_off, 0, kStreamNonTemporal);
+                else __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lvoid *)to, 4, lane_off, wave_off, 0, 0);
             }
         }
     };
     // my tiles: blockIdx.x, blockIdx.x + grid, ...
     const int grid = grid_first;
     const int first = blockIdx.x;
-    const int mine = first < total_tiles ? (total_tiles - first + grid - 1) / grid : 0;
+    // (no grid is wider than its launch has tiles; said here, the first tile's loads need no condition, behind which
+    // the compiler would no longer know how many loads are under way)
+    if (first >= total_tiles) return;
+    const int mine = (total_tiles - first + grid - 1) / grid;
 
     // Segmented sum over aligned groups of `width` lanes (a power of two): row-local DPP moves up
     // to 16 lanes, cross-row permutes beyond.
@@ -952,7 +940,6 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     const bool x_staged = !HALVES || halves_lds_bytes(stage_bytes, x_bytes) <= kLdsBytes;
     uint8_t *xs = x_in_ring ? ring + (kStages - 1) * stage_bytes : ring + kStages * stage_bytes;
     const uint32_t xs0 = x_in_ring ? ring0 + (kStages - 1) * stage_bytes : ring0 + kStages * stage_bytes;
-    int issued = 0;
     if constexpr (!rms && !PACKED) {
         for (int base = 0; x_staged && base < x_bytes; base += nthreads * 16) {
             const int q = base / 16 + tid;
@@ -983,26 +970,31 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     auto load = [&](int base) {
 #pragma unroll
         for (int j = 0; j < kHold; j++) {
-            const int i = base + j * nthreads + tid;
-            v[j] = i < nvec ? xv[i] : float4{0.f, 0.f, 0.f, 0.f};
-            w[j] = i < nvec ? wv[i] : float4{0.f, 0.f, 0.f, 0.f};
+            // (past the end the vector's first columns: under a condition each the loads waited for one another)
+            const int i = base + j * nthreads + tid, from = FULL || i < nvec ? i : 0;
+            v[j] = xv[from];
+            w[j] = wv[from];
         }
     };
     // (these loads go out before the first tile's: a wait for them then leaves the tile in flight
     // while the sum of squares and the products are computed, instead of waiting for it as well)
+    float scale = 0.f;
     if constexpr (rms) {
+        if (p.rms_scale) scale = *p.rms_scale;
         if (held) load(0);
     }
-    for (; issued < kStages - 1 && issued < mine; issued++) issue(first + issued * grid, issued);
+    __builtin_amdgcn_sched_barrier(0);
+    issue(first, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    static_assert(kStages == 2, "one tile is in flight while another is computed");
+    int issued = 1;
     if constexpr (rms) {
-        float scale;
-        if (p.rms_scale) {
-            scale = *p.rms_scale;
-        } else {
+        if (!p.rms_scale) {
             float ss = 0.f;
             if (held) {
 #pragma unroll
                 for (int j = 0; j < kHold; j++) {
+                    if (!FULL && j * nthreads + tid >= nvec) v[j] = float4{0.f, 0.f, 0.f, 0.f};
                     ss = fmaf(v[j].x, v[j].x, ss);
                     ss = fmaf(v[j].y, v[j].y, ss);
                     ss = fmaf(v[j].z, v[j].z, ss);
@@ -1023,8 +1015,9 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
             const uint32_t cell = lds0 + kPartialBytes - 64;
             if (lane == 0) lds_write_b32(cell + wave * 4, __float_as_uint(ss));
             __builtin_amdgcn_s_barrier();
-            ss = 0.f;
-            for (int i = 0; i < nthreads / JL_WAVE; i++) ss += __uint_as_float(lds_read_b32(cell + i * 4));
+            uint32_t sums[4];   // (a launch that normalises has 256 threads)
+            lds_read_x4(cell, sums);
+            ss = ((__uint_as_float(sums[0]) + __uint_as_float(sums[1])) + __uint_as_float(sums[2])) + __uint_as_float(sums[3]);
             scale = (float)(1.0 / sqrt((double)(ss / (float)p.n + p.rms_eps)));
         }
         for (int base = 0; base < nvec; base += nthreads * kHold) {
@@ -1032,7 +1025,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
 #pragma unroll
             for (int j = 0; j < kHold; j++) {
                 const int i = base + j * nthreads + tid;
-                if (i < nvec) {
+                if (FULL || i < nvec) {
                     const floatx4 o = {w[j].x * (scale * v[j].x), w[j].y * (scale * v[j].y),
                                        w[j].z * (scale * v[j].z), w[j].w * (scale * v[j].w)};
                     lds_write_x4(xs0 + ((i >> 4) * 17 + (i & 15)) * 16, o);
@@ -1040,7 +1033,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
             }
         }
     }
-    wait_vm_tiles<L>(issued);
+    JL_WAIT_VM(L);
     __builtin_amdgcn_s_barrier();
 
     float x[64];
@@ -1164,6 +1157,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
     // fill a wave each, so gate/up keeps the LDS hand-over there).
     const bool in_wave = Sp <= (DUAL ? 32 : 64);
     const int r_lds = (DUAL && in_wave) ? (r & 1) * half_rows + (r >> 1) : r;   // tile row this thread reads
+    const int half_gap = (DUAL && r_lds >= half_rows) ? up_at - half_bytes : 0;
     float best = -INFINITY;   // ARGMAX: the largest value this lane has stored, and its row
     int best_at = INT_MAX;
     for (int it = 0; it < mine; it++) {
@@ -1182,8 +1176,8 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         float v = 0.f;
         const uint32_t tile_shift = kShiftedTiles ? (uint32_t)((int64_t)tile * half_bytes) & 15 : 0;   // (one weight)
         if (active) {
-            if constexpr (PACKED) v = slice_dot_lds_packed<TYPE>(ring0 + (it % kStages) * stage_bytes, r_lds, s, row_bytes, px);
-            else v = slice_dot_lds<TYPE>(ring0 + (it % kStages) * stage_bytes + tile_shift, r_lds, s, row_bytes, x, sx);
+            if constexpr (PACKED) v = slice_dot_lds_packed<TYPE>(ring0 + (it % kStages) * stage_bytes + half_gap, r_lds, s, row_bytes, px);
+            else v = slice_dot_lds<TYPE>(ring0 + (it % kStages) * stage_bytes + tile_shift + half_gap, r_lds, s, row_bytes, x, sx);
         }
         if (in_wave) {
             v = group_sum(v, Sp);
@@ -1236,7 +1230,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
             lds_write_b32(lds0 + (it & 1) * kParity + slot * 4, __float_as_uint(v));
         }
     }
-    if (mine > 0 && !in_wave) {
+    if (!in_wave) {
         __builtin_amdgcn_s_barrier();
         finish(first + (mine - 1) * grid, (mine - 1) & 1);
     }
