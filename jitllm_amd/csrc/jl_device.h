@@ -18,6 +18,20 @@ __device__ __forceinline__ float jl_mul_rn(float a, float b) {
     return r;
 }
 
+// WIDTH (16 or 4) bytes per lane from `base` + wave_off + lane_off to LDS, lane by lane behind `to`; only lane_off differs
+// between lanes.  POLICY: cache policy bits (2: non-temporal).
+// A buffer load: one scalar offset per instruction where a global load takes a 64-bit address in two vector registers,
+// and counted by the compiler as any other load, where a global load to LDS (an instruction of the flat family) makes it
+// answer the first use of another loaded value with a wait for everything.
+template <int WIDTH, int POLICY = 0>
+__device__ __forceinline__ void jl_load_to_lds(const void *base, void *to, int lane_off, int wave_off) {
+    typedef __attribute__((address_space(3))) void lds_void;
+    static_assert(WIDTH == 16 || WIDTH == 4, "");
+    const auto from = __builtin_amdgcn_make_buffer_rsrc((void *)base, 0, -1, 0x00020000);
+    if constexpr (WIDTH == 16) __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void *)to, 16, lane_off, wave_off, 0, POLICY);
+    else __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (lds_void *)to, 4, lane_off, wave_off, 0, POLICY);
+}
+
 // IEEE half bits -> float, exact (subnormals included); the device form of Float.float16ToFloat.
 __device__ __forceinline__ float jl_half_bits_to_float(uint32_t bits) {
     return __half2float(__ushort_as_half((unsigned short)(bits & 0xFFFFu)));

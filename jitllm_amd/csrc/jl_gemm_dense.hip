@@ -272,7 +272,12 @@ __device__ __forceinline__ void lds_settle(half8 (&f)[N]) {
 // q|k|v of 3072 or 6144 columns: 256 x 192 in two stages of 56 KB, 128 x 192 in three of 40 KB)
 template <int BM, int BN> constexpr int hh_stages() { return BM + BN >= 448 ? 2 : BM + BN >= 320 ? 3 : 4; }
 
-template <int BM, int BN>
+// How a tile ends; an instance each: one kernel with all three kept scalar registers in vector lanes, and sixteen layers
+// of a 512-token prompt took 2475 us with it and 2459 with three (512 x 2048 over 3072 columns in two runs: 2585 -> 915
+// lines).
+enum Ending { kRows, kSwiglu, kPlanes };   // stored or added to C; gate and up to C; a run's sums to its plane
+
+template <int BM, int BN, Ending END>
 __global__ void __launch_bounds__(512) __attribute__((amdgpu_waves_per_eu(2, 2)))
 jl_gemm_hh(DenseParams p) {
     extern __shared__ __attribute__((aligned(16))) uint8_t lds[];
@@ -303,9 +308,10 @@ jl_gemm_hh(DenseParams p) {
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int lane = tid & 63;
     const int wm = wave / WN, wn = wave % WN;
-    const bool swiglu = p.epilogue == JL_SWIGLU;
-    const int cols_per_tile = swiglu ? BN / 2 : BN;
-    const int ksteps = p.k / DBK / p.splits;   // steps of one work item
+    constexpr bool swiglu = END == kSwiglu;
+    constexpr int cols_per_tile = swiglu ? BN / 2 : BN;
+    const int splits = END == kPlanes ? p.splits : 1;
+    const int ksteps = p.k / DBK / splits;   // steps of one work item
     const uint32_t lds0 = (uint32_t)(uintptr_t)(lvoid *)lds;
 
     // tile order: XCD x (workgroups blockIdx % 8 == x) takes the x-th eighth of the tiles, walked
@@ -325,21 +331,21 @@ jl_gemm_hh(DenseParams p) {
     const int fr = lane & 15, fg = lane >> 4;
     // (row block i of the wave sits 16 rows = 2048 bytes further on with the same swizzle key, so
     // the A fragments need one address register and immediate offsets)
-    uint32_t a_off0, w_off[NB];
+    // (and so do the column blocks of each half of the tile's weights: one address per half in the two-stage tiles,
+    // which have no registers to spare -- the others lose 2 % with it)
+    constexpr int NWO = 2;
+    uint32_t a_off0, w_off[NWO];
     {
         const int r = wm * TM + fr;
         a_off0 = r * 128 + ((fg ^ ((r >> 1) & 7)) << 4);
     }
 #pragma unroll
-    for (int j = 0; j < NB; j++) {
-        const int r = brow[j] + fr;
-        w_off[j] = DBM * 128 + r * 128 + ((fg ^ ((r >> 1) & 7)) << 4);
-    }
+    for (int i = 0; i < 2; i++) w_off[i] = DBM * 128 + (brow[i * NB / 2] + fr) * 128 + ((fg ^ ((fr >> 1) & 7)) << 4);
 
     const uint32_t toff = (uint32_t)(tid >> 3) * (uint32_t)(p.k * 2) + (uint32_t)(((tid & 7) ^ ((tid >> 4) & 7)) << 4);
 
-    for (int item = slot; item < per_xcd * p.splits; item += slots) {
-        const int split = item / per_xcd;
+    for (int item = slot; item < per_xcd * splits; item += slots) {
+        const int split = END == kPlanes ? item / per_xcd : 0;
         const int logical = xcd * per_xcd + (item - split * per_xcd);
         if (logical >= total) continue;
         const int64_t kbytes = (int64_t)split * ksteps * (DBK * 2);   // first column of this run, in bytes
@@ -356,16 +362,12 @@ jl_gemm_hh(DenseParams p) {
         // long, so one 32-bit thread offset serves every slot on top of a uniform address.
         const uint8_t *a_item = (const uint8_t *)(p.A + (int64_t)m0 * p.k) + kbytes;
         const uint8_t *w_item = (const uint8_t *)(p.W + (int64_t)nt * BN * p.k) + kbytes;
-        const int64_t slot_stride = (int64_t)64 * p.k * 2;
+        const int slot_stride = 64 * p.k * 2;
         // load n (of LA + LW) of this thread for stage s
         auto issue_one = [&](int s, int n) {
             uint8_t *dst = lds + (s % NS) * STAGE;
-            if (n < LA)
-                __builtin_amdgcn_global_load_lds((gvoid *)(a_item + n * slot_stride + (int64_t)s * 128 + toff),
-                                                 (lvoid *)(dst + (n * 512 + wave * 64) * 16), 16, 0, 0);
-            else
-                __builtin_amdgcn_global_load_lds((gvoid *)(w_item + (n - LA) * slot_stride + (int64_t)s * 128 + toff),
-                                                 (lvoid *)(dst + DBM * 128 + ((n - LA) * 512 + wave * 64) * 16), 16, 0, 0);
+            if (n < LA) jl_load_to_lds<16>(a_item, dst + (n * 512 + wave * 64) * 16, toff, n * slot_stride + s * 128);
+            else jl_load_to_lds<16>(w_item, dst + DBM * 128 + ((n - LA) * 512 + wave * 64) * 16, toff, (n - LA) * slot_stride + s * 128);
         };
         // after stage s's last load (past the last step: its own line again, so that the count of
         // loads per stage does not change)
@@ -374,8 +376,7 @@ jl_gemm_hh(DenseParams p) {
         auto prefetch = [&](int s) {
             if (wave < PFW) {
                 const int ps = s + PFD < ksteps ? s + PFD : ksteps - 1;
-                __builtin_amdgcn_global_load_lds((gvoid *)(w_item + (int64_t)ps * 128 + pf_off),
-                                                 (lvoid *)(lds + NS * STAGE + wave * 256), 4, 0, 0);
+                jl_load_to_lds<4>(w_item, lds + NS * STAGE + wave * 256, pf_off, ps * 128);
             }
         };
         auto issue = [&](int s) {
@@ -406,7 +407,8 @@ jl_gemm_hh(DenseParams p) {
                 // k-block h: chunk position of chunk (4 h + fg) is the k-block-0 position ^ (4 h)
 #pragma unroll
                 for (int j = 0; j < NB; j++)
-                    asm volatile("ds_read_b128 %0, %1" : "=&v"(fb[h][j]) : "v"((base + w_off[j]) ^ (h << 6)) : "memory");
+                    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=&v"(fb[h][j])
+                                 : "v"((base + w_off[j / (NB / 2)]) ^ (h << 6)), "n"(j % (NB / 2) * 2048) : "memory");
                 const uint32_t aa = (base + a_off0) ^ (h << 6);
 #pragma unroll
                 for (int i = 0; i < MB; i++)
@@ -495,7 +497,7 @@ jl_gemm_hh(DenseParams p) {
         // epilogue: a lane holds four consecutive output columns 4 (lane / 16) .. + 3 of activation
         // row lane % 16 of each block
         const int n0 = nt * cols_per_tile;
-        if (p.splits > 1) {
+        if constexpr (END == kPlanes) {
             // partial sums of this run of K: plain 16-byte stores into the plane of this split; the
             // planes are added in split order and the epilogue applied by the reduce kernel
             const int64_t width = (int64_t)p.ntiles * BN;
@@ -512,11 +514,64 @@ jl_gemm_hh(DenseParams p) {
             }
             continue;
         }
+        // Every value the ending reads is asked for before the first is used (what is added to, some row blocks at a
+        // time): read where they are used, each was a round trip to memory that also waited for the stores before it, MB
+        // NB of them one behind the other.  (Sixteen layers of a 2048-token prompt over a kept copy, whose o and down
+        // projections add 256 tiles of 128 x 128 to C each: 4465 us so, 4225 as it is.)
+        const int mrow = m0 + wm * TM + (lane & 15);
+        float rs[MB];
+        if (p.row_scale) {
+#pragma unroll
+            for (int i = 0; i < MB; i++) rs[i] = p.row_scale[mrow + i * 16];   // (padded to whole tiles)
+        } else {
+#pragma unroll
+            for (int i = 0; i < MB; i++) rs[i] = 1.f;
+        }
+        // (Waited for here, not at a first use behind a condition: the compiler took the loads of one item for possibly
+        // still under way in the loop of the next, whose fragments go to the same registers, and emptied the ring of
+        // stages there after every barrier.)
+#pragma unroll
+        for (int i = 0; i < MB; i++) asm volatile("" : "+v"(rs[i]));
+        const bool quads = n0 + BN <= p.n_total && (p.ldo & 3) == 0 && ((uintptr_t)(p.C + p.col_offset) & 15) == 0;
+        if constexpr (!swiglu) if (quads) {
+            constexpr int CH = NB == 6 ? 2 : MB < 4 ? MB : 4;   // row blocks at a time
+#pragma unroll
+            for (int first = 0; first < MB; first += CH) {
+                float *dst[CH];
+                floatx4 old[CH][NB];
+#pragma unroll
+                for (int i = 0; i < CH; i++) {
+                    const int m = mrow + (first + i) * 16;
+                    dst[i] = p.C + (int64_t)(m < p.rows ? m : p.rows - 1) * p.ldo + p.col_offset + n0 + (lane >> 4) * 4;
+                }
+                if (p.epilogue == JL_RESIDUAL) {
+#pragma unroll
+                    for (int i = 0; i < CH; i++)
+#pragma unroll
+                        for (int j = 0; j < NB; j++) old[i][j] = *(const floatx4 *)(dst[i] + brow[j]);
+#pragma unroll
+                    for (int i = 0; i < CH; i++)
+#pragma unroll
+                        for (int j = 0; j < NB; j++) acc[first + i][j] = old[i][j] + acc[first + i][j] * rs[first + i];
+                } else {
+#pragma unroll
+                    for (int i = 0; i < CH; i++)
+#pragma unroll
+                        for (int j = 0; j < NB; j++) acc[first + i][j] *= rs[first + i];
+                }
+#pragma unroll
+                for (int i = 0; i < CH; i++) {
+                    if (mrow + (first + i) * 16 >= p.rows) continue;
+#pragma unroll
+                    for (int j = 0; j < NB; j++) *(floatx4 *)(dst[i] + brow[j]) = acc[first + i][j];
+                }
+            }
+            continue;
+        }
 #pragma unroll
         for (int i = 0; i < MB; i++) {
-            const int m = m0 + wm * TM + i * 16 + (lane & 15);
+            const int m = mrow + i * 16;
             if (m >= p.rows) continue;
-            const float rs = p.row_scale ? p.row_scale[m] : 1.f;
             float *crow = p.C + (int64_t)m * p.ldo + p.col_offset;
             if (swiglu) {
 #pragma unroll
@@ -524,7 +579,7 @@ jl_gemm_hh(DenseParams p) {
                     const int col = n0 + wn * (TN / 2) + j * 16 + (lane >> 4) * 4;
                     float v[4];
 #pragma unroll
-                    for (int e = 0; e < 4; e++) v[e] = jl_swiglu_rcp(acc[i][j][e] * rs, acc[i][j + NB / 2][e] * rs);
+                    for (int e = 0; e < 4; e++) v[e] = jl_swiglu_rcp(acc[i][j][e] * rs[i], acc[i][j + NB / 2][e] * rs[i]);
                     if (p.c_f16) {
                         jl_store4_f16((_Float16 *)p.C + (int64_t)m * p.ldo + p.col_offset + col, v, p.n_total - col);
                         continue;
@@ -542,7 +597,7 @@ jl_gemm_hh(DenseParams p) {
 #pragma unroll
                 for (int j = 0; j < NB; j++) {
                     const int col = n0 + wn * TN + j * 16 + (lane >> 4) * 4;
-                    float4 v = {acc[i][j][0] * rs, acc[i][j][1] * rs, acc[i][j][2] * rs, acc[i][j][3] * rs};
+                    float4 v = {acc[i][j][0] * rs[i], acc[i][j][1] * rs[i], acc[i][j][2] * rs[i], acc[i][j][3] * rs[i]};
                     float *dst = crow + col;
                     if (col + 3 < p.n_total && (((uintptr_t)dst) & 15) == 0) {
                         if (p.epilogue == JL_RESIDUAL) {
@@ -566,9 +621,9 @@ jl_gemm_hh(DenseParams p) {
     }
 }
 
-template <int BM, int BN>
+template <int BM, int BN, Ending END>
 int launch_dense(jl_context *ctx, const DenseParams &p) {
-    auto fn = jl_gemm_hh<BM, BN>;
+    auto fn = jl_gemm_hh<BM, BN, END>;
     constexpr int lds = hh_stages<BM, BN>() * (BM + BN) * 128 + 1024;   // the ring and the prefetch's landing KB
     static jl_lds_limit_flags configured;
     {
@@ -745,11 +800,14 @@ int jl_launch_gemm_dense(jl_context *ctx, const jl_weight *const *weights, int c
     if (!(bm == 256 || (bm == 128 && bn != 256)) || (bn != 128 && bn != 192 && bn != 256) ||
         (bn == 192 && (swiglu || splits != 1 || n_total % 192 != 0)))
         return jl_fail(JL_ERR_INVALID, "jl_gemm: no %d x %d tile", bm, bn);
-    const int st = bn == 256   ? launch_dense<256, 256>(ctx, p)
-                   : bn == 192 ? (bm == 256 ? launch_dense<256, 192>(ctx, p) : launch_dense<128, 192>(ctx, p))
-                   : bm == 256 ? launch_dense<256, 128>(ctx, p)
-                               : launch_dense<128, 128>(ctx, p);
-    if (st != JL_OK || splits == 1) return st;
+    if (splits == 1) {
+        if (swiglu) return bn == 256 ? launch_dense<256, 256, kSwiglu>(ctx, p) : bm == 256 ? launch_dense<256, 128, kSwiglu>(ctx, p) : launch_dense<128, 128, kSwiglu>(ctx, p);
+        if (bn == 192) return bm == 256 ? launch_dense<256, 192, kRows>(ctx, p) : launch_dense<128, 192, kRows>(ctx, p);
+        return bn == 256 ? launch_dense<256, 256, kRows>(ctx, p) : bm == 256 ? launch_dense<256, 128, kRows>(ctx, p) : launch_dense<128, 128, kRows>(ctx, p);
+    }
+    if (bm != 128 || bn != 128 || swiglu) return jl_fail(JL_ERR_INVALID, "jl_gemm: a %d x %d tile does not cut K", bm, bn);
+    const int st = launch_dense<128, 128, kPlanes>(ctx, p);
+    if (st != JL_OK) return st;
     return jl_launch_gemm_reduce(ctx, planes, row_scale, C, rows, n_total, ntiles,
                                  (int64_t)p.mtiles * bm * ntiles * 128, splits, ldo, col_offset, epilogue);
 }

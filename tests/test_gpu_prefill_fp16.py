@@ -412,3 +412,37 @@ def test_rms_apply_with_the_pending_residual(ctx, rows, n):
     assert np.array_equal(got_x[rows], x[rows])
     assert np.array_equal(scales.get()[:rows].view(np.uint32), want_scales.view(np.uint32))
     assert np.array_equal(out.get().reshape(rows + 1, n)[:rows].view(np.uint16), want.view(np.uint16))
+
+
+@pytest.mark.parametrize("d,T,residual", [
+    (3000, 1024, True),      # 128 x 128 tiles, the last one 56 columns
+    (3000, 1021, False),
+    (6016, 1021, True),      # 256 x 128
+    (3072, 2045, True),      # 128 x 192
+    (6144, 2045, True),      # 256 x 192
+    (8244, 2045, True),      # 256 x 256, the last tile 52 columns
+    (8192, 2048, False),
+])
+def test_tiles_that_end_in_quads_equal_those_that_do_not(ctx, d, T, residual):
+    """The many-row kernel ends a whole tile on 16-byte boundaries with all its reads in front, any other element by
+    element: the same call at an odd column of an odd row length gives the same bits, and rows past the active ones
+    keep theirs."""
+    from jitllm_amd import _lib as L, synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    say("quads", d, T, residual)
+    n, batch = 256, T + 2
+    w = ctx.load_weight(O.Q8_0, synthetic.weight(O.Q8_0, d, n, seed=1790), d, n)
+    x = ctx.half_from_numpy(half_activations((batch, n), 1791))
+    start = synthetic.activations((batch, d), seed=1792)
+    odd = np.full((batch, d + 3), UNTOUCHED, np.float32)
+    odd[:, 1:d + 1] = start
+    proj = QuantizedBatchProjections(ctx, batch, n, d)
+    a, b = ctx.from_numpy(start), ctx.from_numpy(odd)
+    epilogue = L.JL_RESIDUAL if residual else L.JL_STORE
+    proj._gemm([w], x, a, T, d, 0, epilogue)
+    proj._gemm([w], x, b, T, d + 3, 1, epilogue)
+    ctx.sync()
+    a, b = a.get().reshape(batch, d), b.get().reshape(batch, d + 3)
+    assert np.array_equal(a.view(np.uint32), np.ascontiguousarray(b[:, 1:d + 1]).view(np.uint32))
+    assert np.array_equal(a[T:], start[T:]) and not np.array_equal(a[T - 1], start[T - 1])
+    assert (b[:, 0] == UNTOUCHED).all() and (b[:, d + 1:] == UNTOUCHED).all()
