@@ -41,7 +41,6 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x4u __attribute__((ext_vector_type(4), aligned(2)));
-typedef __attribute__((address_space(1))) const void gvoid;
 typedef __attribute__((address_space(1))) const uint8_t gbyte;
 typedef __attribute__((address_space(1))) const u32x4u gpiece;
 typedef __attribute__((address_space(3))) void lvoid;
@@ -320,11 +319,9 @@ jl_gemm_reg(RegParams p) {
         int b = (s >> 1) * KW + kw;
         b = b < nb ? b : nb - 1;
         uint8_t *dst = ring + slot * STAGE;
-        const uint8_t *a = (const uint8_t *)p.A + (int64_t)b * 512 + (s & 1) * 256;
 #pragma unroll
         for (int n = 0; n < LA; n++)
-            __builtin_amdgcn_global_load_lds((gvoid *)(a + a_off[n]),
-                                             (lvoid *)(dst + (n * WN + wn < 4 * MB ? n * WN + wn : 4 * MB - 1) * 1024), 16, 0, 0);
+            jl_load_to_lds<16>(p.A, dst + (n * WN + wn < 4 * MB ? n * WN + wn : 4 * MB - 1) * 1024, a_off[n], b * 512 + (s & 1) * 256);
         asm volatile("" ::: "memory");
     };
 
@@ -525,10 +522,25 @@ jl_gemm_reg(RegParams p) {
 
     // The weight fragment is the matrix instruction's row operand: a lane has output columns 4 g .. of the
     // group for activation row 16 m + r16.
+    // What it reads, the row scales and (where everything lies on 16-byte boundaries) the values it adds to, is asked
+    // for in front of the first store: where they are used each would be a round trip to memory.
+    const bool quads = (p.ldo & 3) == 0 && ((uintptr_t)(p.C + p.col_offset) & 15) == 0 && ((out_col[0] | out_col[NR - 1]) & 3) == 0;
+    const bool adds = quads && p.epilogue == JL_RESIDUAL;
+    constexpr int MINE = (MB + KW - 1) / KW;   // row blocks a set of waves ends
+    float scales[MINE];
+    floatx4 old[MINE][NR];
+#pragma unroll
+    for (int i = 0; i < MINE; i++) {
+        const int at = m0 + 16 * (i * KW + kw) + r16, row = at < p.rows ? at : p.rows - 1;
+        scales[i] = p.row_scale ? p.row_scale[row] : 1.f;
+        if (!adds) continue;
+#pragma unroll
+        for (int j = 0; j < NR; j++) old[i][j] = *(const floatx4 *)(p.C + (int64_t)row * p.ldo + p.col_offset + 4 * g + out_col[j]);
+    }
     auto finish = [&](int m, const floatx4 (&t)[NR]) {
         const int row = m0 + 16 * m + r16;
         if (row >= p.rows) return;
-        const float rs = p.row_scale ? p.row_scale[row] : 1.f;
+        const float rs = scales[m / KW];
         if (rs < 0.f) return;   // (done apart, below)
         const int64_t at = (int64_t)row * p.ldo + p.col_offset + 4 * g;
         if (swiglu) {
@@ -554,8 +566,8 @@ jl_gemm_reg(RegParams p) {
         for (int j = 0; j < NR; j++) {
             float *dst = p.C + at + out_col[j];
             floatx4 v = t[j] * rs;
-            if (out_from[j] == 0 && ((uintptr_t)dst & 15) == 0) {
-                if (p.epilogue == JL_RESIDUAL) v += *(const floatx4 *)dst;
+            if (out_from[j] == 0 && quads) {
+                if (adds) v += old[m / KW][j];
                 *(floatx4 *)dst = v;
             } else {
 #pragma unroll
