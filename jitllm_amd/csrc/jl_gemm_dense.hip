@@ -44,9 +44,8 @@ struct DecodeParams {
                            // t * BN + sel * half + i is row t * half + i of weight sel (0 gate, 1 up)
     int only_own;          // a later pass over weights of mixed types: rows of a weight whose
                            // pointer is null here (another type's, or padding) are left as they are
-    // the call's activations, when they ride along (else virtual_rows = the grid's width):
-    // workgroups blockIdx.x >= virtual_rows convert activation row blockIdx.x - virtual_rows
-    int virtual_rows;
+    int virtual_rows;      // a multiple of kDecodeRows
+    int activation_rows;   // the call's activations, when they ride along: converted by the first workgroups, one a row
     const float *X;        // [rows x k] fp32
     _Float16 *A;           // [padded rows x k]
     float *row_scale;
@@ -71,50 +70,18 @@ __device__ __forceinline__ uint4 pack8_affine(uint32_t q0, uint32_t q1, h2 ds, h
                  __builtin_bit_cast(uint32_t, c), __builtin_bit_cast(uint32_t, e)};
 }
 
-// One thread decodes 8 consecutive columns of one row into one 16-byte store, so a wave writes
-// 1 KB of consecutive fp16 and reads a consecutive run of raw blocks (the 8 quant bytes of a
-// Q8_0 / Q4_0 chunk are only 2-byte aligned; the hardware takes unaligned dword loads).
-// blockIdx.x is the virtual row -- rows that no weight row fills (the end of the last column tile)
-// become zeros -- and blockIdx.y the run of 256 chunks within it.
+// Eight consecutive columns (chunk c) of a row of raw blocks.  (The 8 quant bytes of a Q8_0 / Q4_0 chunk are only
+// 2-byte aligned; the hardware takes unaligned dword loads.)
 struct __attribute__((packed, aligned(2))) Quants8 { uint32_t lo, hi; };
 
 template <int TYPE>
-__global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
-    if ((int)blockIdx.x >= p.virtual_rows) {
-        if (blockIdx.y == 0) jl_row_to_f16(p.X, p.A, p.row_scale, p.rows, p.k, blockIdx.x - p.virtual_rows);
-        return;
-    }
-    const int v = blockIdx.x;
-    const int c = blockIdx.y * 256 + threadIdx.x;   // chunk of 8 columns
-    if (c >= p.k / 8) return;
-    uint4 *dst = (uint4 *)(p.out + (int64_t)v * p.k + c * 8);
-    // (the table is walked with constant indices so that it stays in scalar registers)
-    const uint8_t *w = nullptr;
-    int r = 0;
-    if (p.half) {
-        const int t = v / (2 * p.half), within = v - t * (2 * p.half);
-        const int sel = within >= p.half;
-        r = t * p.half + within - sel * p.half;
-        if (r < p.n_total) w = sel ? p.w[1] : p.w[0];
-    } else {
-#pragma unroll
-        for (int i = 0; i < 8; i++)
-            if (i < p.count && v >= p.begin[i] && v < p.begin[i + 1]) {
-                w = p.w[i];
-                r = v - p.begin[i];
-            }
-    }
-    if (w == nullptr) {
-        if (!p.only_own) *dst = uint4{0, 0, 0, 0};
-        return;
-    }
-    const uint8_t *row = w + (int64_t)r * p.row_bytes;
+__device__ __forceinline__ uint4 decode8(const uint8_t *row, int c) {
     if constexpr (TYPE == JL_Q8_0) {
         const uint8_t *blk = row + (c >> 2) * 34;
         const _Float16 d = *(const _Float16 *)blk;
         const Quants8 q = *(const Quants8 *)(blk + 2 + (c & 3) * 8);
         const h2 bias = {(_Float16)1152.f, (_Float16)1152.f}, d2 = {d, d};
-        *dst = pack8_scaled(q.lo ^ 0x80808080u, q.hi ^ 0x80808080u, bias, d2);
+        return pack8_scaled(q.lo ^ 0x80808080u, q.hi ^ 0x80808080u, bias, d2);
     } else if constexpr (TYPE == JL_Q4_0) {
         // columns 0..15 of a block are the low nibbles of its 16 bytes, 16..31 the high nibbles
         const uint8_t *blk = row + (c >> 2) * 18;
@@ -122,7 +89,7 @@ __global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
         const Quants8 q = *(const Quants8 *)(blk + 2 + (c & 1) * 8);
         const int shift = (c & 2) * 2;
         const h2 bias = {(_Float16)1032.f, (_Float16)1032.f}, d2 = {d, d};
-        *dst = pack8_scaled((q.lo >> shift) & 0x0F0F0F0Fu, (q.hi >> shift) & 0x0F0F0F0Fu, bias, d2);
+        return pack8_scaled((q.lo >> shift) & 0x0F0F0F0Fu, (q.hi >> shift) & 0x0F0F0F0Fu, bias, d2);
     } else if constexpr (TYPE == JL_Q4_1 || TYPE == JL_Q5_0 || TYPE == JL_IQ4_XS) {
         // chunk c % 4 of the group of 32 c / 4: the low (chunks 0, 1) or high (2, 3) nibbles of
         // eight of the group's sixteen bytes; the value is the host decode in fp32 --
@@ -167,7 +134,7 @@ __global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
             else f = jl_mul_rn(a, (float)(int)(int8_t)byte);
             v[e] = (_Float16)f;
         }
-        *dst = *(const uint4 *)v;
+        return *(const uint4 *)v;
     } else if constexpr (TYPE == JL_Q5_K) {
         // chunk c % 32 of super-block c / 32 (d, dmin | 12 scale bytes | qh[32] | qs[128]): sub-block
         // sub, positions pos .. pos + 7; the value is the host decode ((d * sc) * q) - (dmin * m) in
@@ -190,7 +157,7 @@ __global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
             v[e] = (_Float16)__fsub_rn(jl_mul_rn(ds, (float)((q0 >> (8 * e)) & 0xFF)), dm);
             v[4 + e] = (_Float16)__fsub_rn(jl_mul_rn(ds, (float)((q1 >> (8 * e)) & 0xFF)), dm);
         }
-        *dst = *(const uint4 *)v;
+        return *(const uint4 *)v;
     } else if constexpr (TYPE == JL_Q6_K) {
         // chunk c % 32 of super-block c / 32 (ql[128] | qh[64] | 16 signed scales | d): half h,
         // group g, positions pos .. pos + 7 of the group; the value is the host decode
@@ -210,7 +177,7 @@ __global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
             v[e] = (_Float16)jl_mul_rn(ds, (float)((int)((q0 >> (8 * e)) & 0xFF) - 32));
             v[4 + e] = (_Float16)jl_mul_rn(ds, (float)((int)((q1 >> (8 * e)) & 0xFF) - 32));
         }
-        *dst = *(const uint4 *)v;
+        return *(const uint4 *)v;
     } else {
         // sub-block c / 4 of super-block c / 32: low nibbles are the even sub-block of a pair of
         // 32 bytes, high nibbles the odd one
@@ -224,8 +191,68 @@ __global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
         jl_q4k_scale_min(h.y, h.z, h.w, sub, sc, mn);
         const _Float16 ds = (_Float16)(d * (float)sc), dm = (_Float16)(dmin * (float)mn);
         const int shift = (sub & 1) * 4;
-        *dst = pack8_affine((q.x >> shift) & 0x0F0F0F0Fu, (q.y >> shift) & 0x0F0F0F0Fu, h2{ds, ds}, h2{dm, dm});
+        return pack8_affine((q.x >> shift) & 0x0F0F0F0Fu, (q.y >> shift) & 0x0F0F0F0Fu, h2{ds, ds}, h2{dm, dm});
     }
+}
+
+// A wave reads a consecutive run of raw blocks of a row and writes 1 KB of consecutive fp16, a thread 16 bytes of each
+// of kDecodeRows rows, all of whose loads are under way before the first store.
+// blockIdx.x: the call's activation rows, where they ride along -- they begin first, a row's two passes are a longer
+// chain than a decode --, then sets of virtual rows, of which those that no weight row fills (the end of the last
+// column tile) become zeros; blockIdx.y is the run of 256 chunks within a row.
+constexpr int kDecodeRows = 4;
+
+template <int TYPE>
+__global__ void __launch_bounds__(256) jl_decode_to_f16(DecodeParams p) {
+    if ((int)blockIdx.x < p.activation_rows) {
+        if (blockIdx.y == 0) jl_row_to_f16(p.X, p.A, p.row_scale, p.rows, p.k, blockIdx.x);
+        return;
+    }
+    const int first = (blockIdx.x - p.activation_rows) * kDecodeRows;
+    const int c = blockIdx.y * 256 + threadIdx.x;   // chunk of 8 columns
+    if (c >= p.k / 8) return;
+    // the weight row of a virtual row, and how many of its weight are left from it on
+    // (the table is walked with constant indices so that it stays in scalar registers)
+    auto row_of = [&](int v, int &left) -> const uint8_t * {
+        const uint8_t *w = nullptr;
+        int r = 0;
+        left = 0;
+        if (p.half) {
+            const int t = v / (2 * p.half), within = v - t * (2 * p.half);
+            const int sel = within >= p.half;
+            r = t * p.half + within - sel * p.half;
+            if (r < p.n_total) {
+                w = sel ? p.w[1] : p.w[0];
+                left = p.n_total - r < (1 + sel) * p.half - within ? p.n_total - r : (1 + sel) * p.half - within;
+            }
+        } else {
+#pragma unroll
+            for (int i = 0; i < 8; i++)
+                if (i < p.count && v >= p.begin[i] && v < p.begin[i + 1]) {
+                    w = p.w[i];
+                    r = v - p.begin[i];
+                    left = p.begin[i + 1] - v;
+                }
+        }
+        return w ? w + (int64_t)r * p.row_bytes : nullptr;
+    };
+    int left;
+    const uint8_t *row[kDecodeRows];
+    row[0] = row_of(first, left);
+    if (row[0] && left >= kDecodeRows) {
+#pragma unroll
+        for (int i = 1; i < kDecodeRows; i++) row[i] = row[0] + (int64_t)i * p.row_bytes;
+    } else {
+#pragma unroll
+        for (int i = 1; i < kDecodeRows; i++) row[i] = row_of(first + i, left);
+    }
+    uint4 out[kDecodeRows];
+#pragma unroll
+    for (int i = 0; i < kDecodeRows; i++) out[i] = row[i] ? decode8<TYPE>(row[i], c) : uint4{0, 0, 0, 0};
+    _Float16 *dst = p.out + (int64_t)first * p.k + c * 8;
+#pragma unroll
+    for (int i = 0; i < kDecodeRows; i++)
+        if (row[i] || !p.only_own) *(uint4 *)(dst + (int64_t)i * p.k) = out[i];
 }
 
 // ---- fp16 GEMM ----------------------------------------------------------------------------------
@@ -639,9 +666,9 @@ int launch_dense(jl_context *ctx, const DenseParams &p) {
 }
 
 template <int TYPE>
-int launch_decode(jl_context *ctx, const DecodeParams &d, int activation_rows) {
+int launch_decode(jl_context *ctx, const DecodeParams &d) {
     hipLaunchKernelGGL(jl_decode_to_f16<TYPE>,
-                       dim3((unsigned)(d.virtual_rows + activation_rows), (unsigned)((d.k / 8 + 255) / 256)),
+                       dim3((unsigned)(d.virtual_rows / kDecodeRows + d.activation_rows), (unsigned)((d.k / 8 + 255) / 256)),
                        dim3(256), 0, ctx->stream, d);
     JL_HIP(hipGetLastError());
     return JL_OK;
@@ -764,18 +791,18 @@ int jl_launch_gemm_dense(jl_context *ctx, const jl_weight *const *weights, int c
             if (weights[j]->type != pass_type) pass.w[j] = nullptr;
         pass.row_bytes = k / jl_block_elems(pass_type) * jl_block_bytes(pass_type);
         pass.only_own = first_pass ? 0 : 1;
-        const int ride = first_pass ? xr : 0;
+        pass.activation_rows = first_pass ? xr : 0;
         first_pass = false;
         int dst;
         switch (pass_type) {
-            case JL_Q8_0: dst = launch_decode<JL_Q8_0>(ctx, pass, ride); break;
-            case JL_Q4_0: dst = launch_decode<JL_Q4_0>(ctx, pass, ride); break;
-            case JL_Q4_K: dst = launch_decode<JL_Q4_K>(ctx, pass, ride); break;
-            case JL_Q5_K: dst = launch_decode<JL_Q5_K>(ctx, pass, ride); break;
-            case JL_Q6_K: dst = launch_decode<JL_Q6_K>(ctx, pass, ride); break;
-            case JL_Q4_1: dst = launch_decode<JL_Q4_1>(ctx, pass, ride); break;
-            case JL_Q5_0: dst = launch_decode<JL_Q5_0>(ctx, pass, ride); break;
-            case JL_IQ4_XS: dst = launch_decode<JL_IQ4_XS>(ctx, pass, ride); break;
+            case JL_Q8_0: dst = launch_decode<JL_Q8_0>(ctx, pass); break;
+            case JL_Q4_0: dst = launch_decode<JL_Q4_0>(ctx, pass); break;
+            case JL_Q4_K: dst = launch_decode<JL_Q4_K>(ctx, pass); break;
+            case JL_Q5_K: dst = launch_decode<JL_Q5_K>(ctx, pass); break;
+            case JL_Q6_K: dst = launch_decode<JL_Q6_K>(ctx, pass); break;
+            case JL_Q4_1: dst = launch_decode<JL_Q4_1>(ctx, pass); break;
+            case JL_Q5_0: dst = launch_decode<JL_Q5_0>(ctx, pass); break;
+            case JL_IQ4_XS: dst = launch_decode<JL_IQ4_XS>(ctx, pass); break;
             default: return jl_fail(JL_ERR_UNSUPPORTED, "jl_gemm: no kernel for a ggml type %d weight", pass_type);
         }
         if (dst != JL_OK) return dst;
