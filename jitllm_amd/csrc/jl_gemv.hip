@@ -867,9 +867,8 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
         const uint8_t *base = wseg + (offset - shift);
         const uint8_t *base_up = DUAL ? w_up_first + offset : base;
         uint8_t *dst = ring + st * stage_bytes;
-        const bool whole = exact && (FULL || bytes == half_bytes);  // uniform
-#pragma unroll
-        for (int k = 0; k < L; k++) {
+        // `whole`: every slot is inside the tile, nothing to redirect
+        auto load = [&](int k, bool whole) __attribute__((always_inline)) {
             const int width = k < X4 ? 16 : 4;
             // the wave's place among the loads of this width, and where those begin
             int unit = k < X4 ? k * nwaves + wave : wave;
@@ -884,8 +883,7 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
             // (a shifted tile's last 16 bytes may run past its end, not past the weight's, whose
             // bytes are a multiple of 16)
             const int off = at + lane * width;
-            const bool real = whole || (kShiftedTiles ? off < bytes : off + width <= bytes);
-            // the usual case (uniform): every slot is inside the tile, nothing to redirect
+            const bool real = kShiftedTiles ? off < bytes : off + width <= bytes;
             const int lane_off = whole ? lane * width : real ? off : 0, wave_off = whole ? at : 0;
             if (k < X4) {
                 if (DUAL && whole) jl_load_to_lds<16, kStreamNonTemporal>(from, to, lane_off, wave_off);
@@ -894,6 +892,14 @@ __global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first,
                 if (DUAL && whole) jl_load_to_lds<4, kStreamNonTemporal>(from, to, lane_off, wave_off);
                 else jl_load_to_lds<4>(from, to, lane_off, wave_off);
             }
+        };
+        // (a branch, not a choice per load: 4025 x 1024 Q8_0, a general instance, 3.42 us so and 3.55 with choices)
+        if (exact && (FULL || bytes == half_bytes)) {   // uniform, the usual case
+#pragma unroll
+            for (int k = 0; k < L; k++) load(k, true);
+        } else {
+#pragma unroll
+            for (int k = 0; k < L; k++) load(k, false);
         }
     };
     // my tiles: blockIdx.x, blockIdx.x + grid, ...
