@@ -9,7 +9,7 @@
 //
 //   jl_decode_to_f16   raw blocks -> [virtual rows x K] fp16, the host decode rounded once to fp16
 //                      (bit for bit what the fused kernel multiplies with); one launch per call
-//   jl_gemm_hh<BM, BN> C = A16 . W16^T on v_mfma_f32_16x16x32_f16, BM x BN tiles (256 x 256, 256 x 192,
+//   jl_gemm_hh         C = A16 . W16^T on v_mfma_f32_16x16x32_f16, BM x BN tiles (256 x 256, 256 x 192,
 //                      256 x 128, 128 x 192, 128 x 128) in steps of 64 columns; eight waves that each bring in their
 //                      share of both operands by LDS-DMA, the two waves of a SIMD half a step apart
 #include "jl_device.h"

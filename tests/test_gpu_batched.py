@@ -1173,3 +1173,29 @@ def test_mixed_types_side_by_side_below_512_rows_are_their_runs(ctx, rows):
     for w in (wq, wk, wv):
         w.free()
     proj.workspace.free()
+
+
+@pytest.mark.parametrize("types,dims", [
+    ((O.Q8_0, O.Q8_0, O.Q8_0), (257, 129, 255)),     # every boundary inside a pair of decoded rows
+    ((O.Q4_0, O.Q4_0, O.Q4_0), (33, 1, 64)),         # a weight of one row between two
+    ((O.Q8_0, O.Q4_0, O.Q8_0), (129, 63, 65)),       # a pass per type, each leaving the other's rows alone
+])
+def test_weights_of_odd_row_counts_decoded_side_by_side(ctx, types, dims):
+    """The pass that decodes a call's weights takes two virtual rows to a thread: pairs across the boundary of two
+    weights, and activations that ride along."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    n, T = 320, 9     # (no whole 256-column blocks: decoded at any row count)
+    say("odd rows side by side", types, dims)
+    raws = [synthetic.weight(t, d, n, seed=1810 + i) for i, (t, d) in enumerate(zip(types, dims))]
+    ws = [ctx.load_weight(t, raw, d, n) for t, raw, d in zip(types, raws, dims)]
+    X = synthetic.activations((T, n), seed=1813)
+    out = ctx.from_numpy(np.full((T, sum(dims)), UNTOUCHED, np.float32))
+    QuantizedBatchProjections(ctx, T, n, sum(dims)).fusedQKV(ctx.from_numpy(X), out, *ws, activeRows=T)
+    ctx.sync()
+    got = out.get().reshape(T, -1)
+    at = 0
+    for t, raw, d in zip(types, raws, dims):
+        ref = O.matmul_batch(t, raw, X, d, n)
+        assert rel_err(got[:, at:at + d], ref, magnitude(t, raw, X, d, n)) < F16_BOUND
+        at += d
