@@ -393,9 +393,16 @@ jl_gemm_hh(DenseParams p) {
         const uint8_t *w_item = (const uint8_t *)(p.W + (int64_t)nt * BN * p.k) + kbytes;
         const int slot_stride = 64 * p.k * 2;
         // load n (of LA + LW) of this thread for stage s
+        // (global loads in the two-stage tiles, buffer loads in the others: gate/up 2 x [8192 x 3072] at 1663 rows 172 us
+        // with buffer loads and 159 with global ones, eight layers of a 2048-token prompt of an 8B Q4_K file 6658 and
+        // 6570; the smaller tiles gain 1 - 2 % from the vector registers that 64-bit addresses took)
         auto issue_one = [&](int s, int n) {
             uint8_t *dst = lds + (s % NS) * STAGE;
-            if (n < LA) jl_load_to_lds<16>(a_item, dst + (n * 512 + wave * 64) * 16, toff, n * slot_stride + s * 128);
+            if constexpr (NS == 2) {
+                const uint8_t *src = n < LA ? a_item + (int64_t)n * slot_stride : w_item + (int64_t)(n - LA) * slot_stride;
+                uint8_t *to = n < LA ? dst + n * 8192 : dst + DBM * 128 + (n - LA) * 8192;
+                __builtin_amdgcn_global_load_lds((gvoid *)(src + (int64_t)s * 128 + toff), (lvoid *)(to + wave * 1024), 16, 0, 0);
+            } else if (n < LA) jl_load_to_lds<16>(a_item, dst + (n * 512 + wave * 64) * 16, toff, n * slot_stride + s * 128);
             else jl_load_to_lds<16>(w_item, dst + DBM * 128 + ((n - LA) * 512 + wave * 64) * 16, toff, (n - LA) * slot_stride + s * 128);
         };
         // after stage s's last load (past the last step: its own line again, so that the count of
@@ -405,7 +412,8 @@ jl_gemm_hh(DenseParams p) {
         auto prefetch = [&](int s) {
             if (wave < PFW) {
                 const int ps = s + PFD < ksteps ? s + PFD : ksteps - 1;
-                jl_load_to_lds<4>(w_item, lds + NS * STAGE + wave * 256, pf_off, ps * 128);
+                __builtin_amdgcn_global_load_lds((gvoid *)(w_item + (int64_t)ps * 128 + pf_off),
+                                                 (lvoid *)(lds + NS * STAGE + wave * 256), 4, 0, 0);
             }
         };
         auto issue = [&](int s) {
