@@ -20,6 +20,7 @@ namespace {
 
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(1))) const void gvoid;
+typedef __attribute__((address_space(1))) const uint8_t gbyte;
 typedef __attribute__((address_space(3))) void lvoid;
 
 #define JL_WAIT_VM(N) \
@@ -392,18 +393,21 @@ jl_gemm_hh(DenseParams p) {
         const uint8_t *a_item = (const uint8_t *)(p.A + (int64_t)m0 * p.k) + kbytes;
         const uint8_t *w_item = (const uint8_t *)(p.W + (int64_t)nt * BN * p.k) + kbytes;
         const int slot_stride = 64 * p.k * 2;
-        // load n (of LA + LW) of this thread for stage s
-        // (global loads in the two-stage tiles, buffer loads in the others: gate/up 2 x [8192 x 3072] at 1663 rows 172 us
-        // with buffer loads and 159 with global ones, eight layers of a 2048-token prompt of an 8B Q4_K file 6658 and
-        // 6570; the smaller tiles gain 1 - 2 % from the vector registers that 64-bit addresses took)
+        // load n (of LA + LW) of this thread for stage s.
+        // The address is a scalar one and `at` a copy: left to itself the compiler adds the two up to a 64-bit address in
+        // vector registers for every load, and keeps up to 33 scalars in vector lanes for it (jl_load_to_lds says why buffer
+        // loads elsewhere).  Buffer loads need no more registers than this, but hold their wave at issue where the rows lie
+        // no power of two apart and come from HBM -- gate/up 2 x [13824 x 2560] at 524 rows, 256 x 128 tiles: 138 us with
+        // them, 117 so, of the same requests, hits and misses, and 54.7 against 39.1 million wave cycles of
+        // SQ_WAIT_INST_ANY; x 2048 92.8 and 92.6.  Over 143 calls of 1536 ... 13824 columns the time is 15 % less to 2 % more.
         auto issue_one = [&](int s, int n) {
             uint8_t *dst = lds + (s % NS) * STAGE;
-            if constexpr (NS == 2) {
-                const uint8_t *src = n < LA ? a_item + (int64_t)n * slot_stride : w_item + (int64_t)(n - LA) * slot_stride;
-                uint8_t *to = n < LA ? dst + n * 8192 : dst + DBM * 128 + (n - LA) * 8192;
-                __builtin_amdgcn_global_load_lds((gvoid *)(src + (int64_t)s * 128 + toff), (lvoid *)(to + wave * 1024), 16, 0, 0);
-            } else if (n < LA) jl_load_to_lds<16>(a_item, dst + (n * 512 + wave * 64) * 16, toff, n * slot_stride + s * 128);
-            else jl_load_to_lds<16>(w_item, dst + DBM * 128 + ((n - LA) * 512 + wave * 64) * 16, toff, (n - LA) * slot_stride + s * 128);
+            const uint8_t *src = (n < LA ? a_item + (int64_t)n * slot_stride : w_item + (int64_t)(n - LA) * slot_stride) + (int64_t)s * 128;
+            uint8_t *to = n < LA ? dst + n * 8192 : dst + DBM * 128 + (n - LA) * 8192;
+            asm("" : "+s"(src));
+            uint32_t at;
+            asm("" : "=v"(at) : "0"(toff));
+            __builtin_amdgcn_global_load_lds((gvoid *)((gbyte *)src + at), (lvoid *)(to + wave * 1024), 16, 0, 0);
         };
         // after stage s's last load (past the last step: its own line again, so that the count of
         // loads per stage does not change)
