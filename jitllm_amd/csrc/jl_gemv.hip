@@ -731,6 +731,16 @@ __device__ __forceinline__ uintptr_t uniform_value(uintptr_t v) {
     return v;
 }
 
+// Waves a SIMD must hold, so that the compiler counts registers for them.  Q4_K's plain and norm-folding instances for rows
+// of one weight fit 96 registers and five waves, and where the LDS has room for five workgroups (rows of 768 and of 1280
+// ... 1792 columns) the grid is that wide; left alone they take 105, the grid is a fifth narrower (8960 x 768 3.55 us so and
+// 3.38 with five, 151936 x 1536 32.2 and 31.3), and where the LDS holds four they are no faster either (4096 x 2560 4.20 and
+// 4.10, 3584 x 3584 4.52 and 4.45).  Rows that fill sixteen slices have always taken 104: not held down.  Q8_0 instances of
+// 97, held to 96, lose up to a fifth of their speed (24576 x 2560 15.2 -> 18.6), and the LDS holds four of theirs.
+template <int TYPE>
+constexpr int least_waves(bool dual, bool packed, int threads, int spt, bool segs, bool part, bool argmax) {
+    return TYPE == JL_Q4_K && !dual && !packed && threads == 256 && !segs && !argmax && (spt == 32 || spt == 64 || (spt == 16 && part)) ? 5 : 1;
+}
 
 // SPT != 0 is the kernel for the usual launch, with its geometry known to the compiler: rows of
 // exactly SPT slices (a power of two), THREADS / SPT rows per tile and, in every segment, a row
@@ -755,7 +765,8 @@ __device__ __forceinline__ uintptr_t uniform_value(uintptr_t v) {
 // partial sums.)
 template <int TYPE, bool DUAL, bool RMS, bool PACKED = false, int THREADS = 256, int SPT = 0, bool SEGS = false,
           bool PART = false, bool ARGMAX = false, bool HALVES = false>
-__global__ void __launch_bounds__(THREADS) jl_gemv_tiles(const uint8_t *w_first, const uint8_t *w_up_first, const float *x_first, int tiles_first,
+__global__ void __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(least_waves<TYPE>(DUAL, PACKED, THREADS, SPT, SEGS, PART, ARGMAX))))
+jl_gemv_tiles(const uint8_t *w_first, const uint8_t *w_up_first, const float *x_first, int tiles_first,
               int rows_first, int grid_first, int S_first, int row_bytes_first, int shape_first,
               const float *rms_w_first, GemvParams p) {
     // The leading arguments repeat what the kernel needs before its first tile's loads can go out
