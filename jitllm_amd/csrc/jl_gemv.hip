@@ -1395,6 +1395,12 @@ template <int TYPE, bool DUAL, bool RMS, bool PACKED = false, int THREADS = 256,
 int launch_tiles_of(jl_context *ctx, const GemvParams &p, int threads, int lds, int *cells = nullptr) {
     auto fn = jl_gemv_tiles<TYPE, DUAL, RMS, PACKED, THREADS, SPT, SEGS, PART, ARGMAX, HALVES>;
     int per_cu = blocks_per_cu((const void *)fn, ctx->device, threads, lds);
+    // Gate/up of Q8_0, Q4_0 and Q6_K takes three workgroups a compute unit where registers and LDS hold four: fewer heads
+    // for the same tiles, and memory is as busy.  Four and three (the first two with their norms): Q8_0 2 x [8192 x 2048]
+    // 9.40 and 8.73 us, 2 x [8960 x 896] 7.03 and 6.09, Q4_0 2 x [5120 x 1280] 6.12 and 5.69, 2 x [8192 x 2048] 7.50 and
+    // 6.85, Q6_K 2 x [8192 x 2048] 8.60 and 7.85; Q4_0 2 x [8960 x 1536] 7.77 and 7.86, Q8_0 2 x [9728 x 2560] 13.44 and
+    // 13.89; other sizes within 1 %.  The other types': not tried.
+    if (DUAL && !PACKED && (TYPE == JL_Q8_0 || TYPE == JL_Q4_0 || TYPE == JL_Q6_K)) per_cu = std::min(per_cu, 3);
     int total = p.seg_tile_begin[p.nseg];
     int grid = ctx->compute_units * per_cu;
     if (grid > total) grid = total;
