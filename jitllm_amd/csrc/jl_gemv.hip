@@ -967,7 +967,7 @@ jl_gemv_tiles(const uint8_t *w_first, const uint8_t *w_up_first, const float *x_
     // The workgroup reads x and the weights with coalesced 16-byte loads and leaves the
     // product in the LDS region the plain path fills with x, so everything after is shared
     // and the LDS footprint (workgroups per compute unit) is that of the plain path.
-    const int nvec = rms ? p.n / 4 : 0;
+    const int nvec = rms ? S * 16 : 0;
     const float4 *xv = (const float4 *)x_first, *wv = (const float4 *)rms_w_first;
     // rows of up to kHold x 4 x nthreads columns are read once and held in registers from the
     // sum of squares to the product; longer ones are read again for the product (the
@@ -989,15 +989,20 @@ jl_gemv_tiles(const uint8_t *w_first, const uint8_t *w_up_first, const float *x_
     // tiles came in by global loads to LDS (jl_load_to_lds): a token of the 7B Q4_K_M model 1498 us, now 1471)
     float scale = 0.f;
     if constexpr (rms) {
-        if (p.rms_scale) scale = *p.rms_scale;
         if (held) load(0);
     }
     __builtin_amdgcn_sched_barrier(0);
     issue(first, 0);
     __builtin_amdgcn_sched_barrier(0);
     static_assert(kStages == 2, "one tile is in flight while another is computed");
+    // What is still to come from the argument buffer, behind the loads and in one trip.  Nothing in front of them may wait
+    // for it: with the scale's address read there, Q8_0 32000 x 2048 with its norm and argmax took 18.22 us, q|k|v 3072 x
+    // 2048 4.53; 17.60 and 3.79 so (17.75 and 4.98 when neither read nor buffer loads were there).
+    if constexpr (rms) asm volatile("" : : "s"(p.rms_scale), "s"(p.rms_eps), "s"(p.n), "s"(SEGS ? seg_out[1] : out0), "s"(p.epilogue));
     if constexpr (rms) {
-        if (!p.rms_scale) {
+        if (p.rms_scale) {
+            scale = *(const __attribute__((address_space(4))) float *)p.rms_scale;   // (a scalar load: the tile stays in flight)
+        } else {
             float ss = 0.f;
             if (held) {
 #pragma unroll
