@@ -400,13 +400,17 @@ jl_gemm_hh(DenseParams p) {
         // no power of two apart and come from HBM -- gate/up 2 x [13824 x 2560] at 524 rows, 256 x 128 tiles: 138 us with
         // them, 117 so, of the same requests, hits and misses, and 54.7 against 39.1 million wave cycles of
         // SQ_WAIT_INST_ANY; x 2048 92.8 and 92.6.  Over 143 calls of 1536 ... 13824 columns the time is 15 % less to 2 % more.
+        // (256 x 256 is left to the compiler: a copy more and 12 - 17 vector registers go to memory instead of 6 - 8, gate/up
+        // 2 x [18944 x 3584] at 950 rows 269.6 us and 266.8, 2 x [12288 x 4096] at 1306 rows 309.9 and 306.2, others the same)
         auto issue_one = [&](int s, int n) {
             uint8_t *dst = lds + (s % NS) * STAGE;
             const uint8_t *src = (n < LA ? a_item + (int64_t)n * slot_stride : w_item + (int64_t)(n - LA) * slot_stride) + (int64_t)s * 128;
             uint8_t *to = n < LA ? dst + n * 8192 : dst + DBM * 128 + (n - LA) * 8192;
-            asm("" : "+s"(src));
-            uint32_t at;
-            asm("" : "=v"(at) : "0"(toff));
+            uint32_t at = toff;
+            if constexpr (BM + BN < 512) {
+                asm("" : "+s"(src));
+                asm("" : "=v"(at) : "0"(toff));
+            }
             __builtin_amdgcn_global_load_lds((gvoid *)((gbyte *)src + at), (lvoid *)(to + wave * 1024), 16, 0, 0);
         };
         // after stage s's last load (past the last step: its own line again, so that the count of
