@@ -302,9 +302,9 @@ __device__ __forceinline__ void lds_settle(half8 (&f)[N]) {
 // q|k|v of 3072 or 6144 columns: 256 x 192 in two stages of 56 KB, 128 x 192 in three of 40 KB)
 template <int BM, int BN> constexpr int hh_stages() { return BM + BN >= 448 ? 2 : BM + BN >= 320 ? 3 : 4; }
 
-// How a tile ends; an instance each: one kernel with all three kept scalar registers in vector lanes, and sixteen layers
-// of a 512-token prompt took 2475 us with it and 2459 with three (512 x 2048 over 3072 columns in two runs: 2585 -> 915
-// lines).
+// How a tile ends; an instance each: one kernel with all three wanted more scalar registers than there are, and sixteen
+// layers of a 512-token prompt took 2475 us with it and 2459 with three (512 x 2048 over 3072 columns in two runs: 2585 ->
+// 915 lines).  (256 x 256 keeps 25 - 33 scalars in vector lanes all the same; the others none.)
 enum Ending { kRows, kSwiglu, kPlanes };   // stored or added to C; gate and up to C; a run's sums to its plane
 
 template <int BM, int BN, Ending END>
@@ -361,10 +361,9 @@ jl_gemm_hh(DenseParams p) {
     const int fr = lane & 15, fg = lane >> 4;
     // (row block i of the wave sits 16 rows = 2048 bytes further on with the same swizzle key, so
     // the A fragments need one address register and immediate offsets)
-    // (and so do the column blocks of each half of the tile's weights: one address per half in the two-stage tiles,
-    // which have no registers to spare -- the others lose 2 % with it)
-    constexpr int NWO = 2;
-    uint32_t a_off0, w_off[NWO];
+    // (and so do the column blocks of each half of the wave's weights, which a SwiGLU tile takes from its two halves: an
+    // address for each -- one for every column block costs four to six registers and 0.4 % of the time, the mean of 62 calls)
+    uint32_t a_off0, w_off[2];
     {
         const int r = wm * TM + fr;
         a_off0 = r * 128 + ((fg ^ ((r >> 1) & 7)) << 4);
@@ -579,7 +578,8 @@ jl_gemm_hh(DenseParams p) {
         for (int i = 0; i < MB; i++) asm volatile("" : "+v"(rs[i]));
         const bool quads = n0 + BN <= p.n_total && (p.ldo & 3) == 0 && ((uintptr_t)(p.C + p.col_offset) & 15) == 0;
         if constexpr (!swiglu) if (quads) {
-            constexpr int CH = NB == 6 ? 2 : MB < 4 ? MB : 4;   // row blocks at a time
+            // row blocks at a time: what they add to takes up to 64 registers, those of the fragments (6 x 3 would be 72)
+            constexpr int CH = NB == 6 ? 2 : MB < 4 ? MB : 4;
 #pragma unroll
             for (int first = 0; first < MB; first += CH) {
                 float *dst[CH];

@@ -313,6 +313,9 @@ jl_gemm_reg(RegParams p) {
     }
     // step s = half s % 2 of block (s / 2) KW + kw; steps past the last one: that one again, so that the count
     // of loads does not change
+    // (Buffer loads: 141 calls of 65 ... 511 rows, all four types, take 0.8 % less time with them than with global ones,
+    // 0.2 % more in the worst of 28 pairs of type and tiling.  What they bring in lies in the caches, where how far apart rows
+    // are does not matter to them; it does in jl_gemm_hh, which has global ones.)
     const int last_step = 2 * iters - 1;
     auto issue_stage = [&](int s, int slot) {
         s = s < last_step ? s : last_step;

@@ -487,9 +487,9 @@ __device__ __forceinline__ float slice_dot_packed_q4_k(const uint4 &h, const uin
 
 // ---- LDS access by hand ----------------------------------------------------------------------
 //
-// The tile stages are filled by LDS-DMA loads (global_load_lds_*), which the compiler tracks only
-// coarsely: any LDS read it can see makes it wait for every outstanding vector-memory operation,
-// which would drain the prefetch pipeline each tile.  All LDS traffic of the kernel therefore goes
+// The tile stages are filled by LDS-DMA loads (jl_load_to_lds; the activation vector by global_load_lds_*), which
+// the compiler tracks only coarsely: any LDS read it can see makes it wait for every outstanding vector-memory
+// operation, which would drain the prefetch pipeline each tile.  All LDS traffic of the kernel therefore goes
 // through inline assembly with explicit waits, and the workgroup barrier is the bare instruction.
 
 typedef __attribute__((address_space(1))) const void gvoid;
