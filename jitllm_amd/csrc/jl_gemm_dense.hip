@@ -845,6 +845,7 @@ int jl_launch_gemm_dense(jl_context *ctx, const jl_weight *const *weights, int c
     if (!(bm == 256 || (bm == 128 && bn != 256)) || (bn != 128 && bn != 192 && bn != 256) ||
         (bn == 192 && (swiglu || splits != 1 || n_total % 192 != 0)))
         return jl_fail(JL_ERR_INVALID, "jl_gemm: no %d x %d tile", bm, bn);
+    ctx->last_tile.store(bm * 1000 + bn, std::memory_order_relaxed);
     if (splits == 1) {
         if (swiglu) return bn == 256 ? launch_dense<256, 256, kSwiglu>(ctx, p) : bm == 256 ? launch_dense<256, 128, kSwiglu>(ctx, p) : launch_dense<128, 128, kSwiglu>(ctx, p);
         if (bn == 192) return bm == 256 ? launch_dense<256, 192, kRows>(ctx, p) : launch_dense<128, 192, kRows>(ctx, p);

@@ -30,12 +30,15 @@ struct jl_context {
     bool split_k = true;
     // the kernel of the last batched projection, one of JL_GEMM_*, for the tests (jl_context_last_gemm)
     std::atomic<int> last_gemm{0};
+    // rows * 1000 + columns of the tile of the last call that jl_gemm_hh took, for the tests (jl_context_last_tile)
+    std::atomic<int> last_tile{0};
 };
 #define JL_GEMM_STREAMED 1          // jl_gemm_skinny
 #define JL_GEMM_IN_LOOP 2           // jl_gemm_f16
 #define JL_GEMM_DECODED 3           // jl_gemm_hh
 #define JL_GEMM_IN_REGISTERS 100    // jl_gemm_reg: this and the number of its tiling
 extern "C" int jl_context_last_gemm(const jl_context *ctx);
+extern "C" int jl_context_last_tile(const jl_context *ctx);
 #define JL_CONTEXT_SCRATCH_BYTES 8192
 #define JL_CONTEXT_ARRIVALS 1024
 #define JL_BOUNCE_HALF_BYTES (8u << 20)

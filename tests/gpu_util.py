@@ -22,6 +22,11 @@ def last_gemm(ctx) -> int:
     return ctx._lib.jl_context_last_gemm(ctx.handle)
 
 
+def last_tile(ctx) -> tuple:
+    """(rows, columns) of the tile that the last call of the many-row kernel took."""
+    return divmod(ctx._lib.jl_context_last_tile(ctx.handle), 1000)
+
+
 def magnitude(t: int, raw: np.ndarray, X: np.ndarray, d: int, n: int) -> np.ndarray:
     """sum_j |w_ij x_bj| in float64, [B x d] (or [d] for a vector)."""
     w = np.abs(NP.DEQUANT[t](raw).reshape(d, n).astype(np.float64))

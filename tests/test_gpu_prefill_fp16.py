@@ -7,7 +7,7 @@ import ctypes as C
 import numpy as np
 import pytest
 
-from gpu_util import magnitude, rel_err, say
+from gpu_util import last_tile, magnitude, rel_err, say
 from oracle import pyoracle as O
 
 pytestmark = pytest.mark.gpu
@@ -414,16 +414,20 @@ def test_rms_apply_with_the_pending_residual(ctx, rows, n):
     assert np.array_equal(out.get().reshape(rows + 1, n)[:rows].view(np.uint16), want.view(np.uint16))
 
 
-@pytest.mark.parametrize("d,T,residual", [
-    (3000, 1024, True),      # 128 x 128 tiles, the last one 56 columns
-    (3000, 1021, False),
-    (6016, 1021, True),      # 256 x 128
-    (3072, 2045, True),      # 128 x 192
-    (6144, 2045, True),      # 256 x 192
-    (8244, 2045, True),      # 256 x 256, the last tile 52 columns
-    (8192, 2048, False),
+# (the tile is the one that 256 compute units are priced to)
+@pytest.mark.parametrize("d,T,residual,tile", [
+    (3000, 1024, True, (128, 128)),      # the last tile 56 columns
+    (3000, 1021, False, (128, 128)),
+    (6016, 1021, True, (256, 128)),
+    (3072, 2045, True, (128, 192)),
+    (6144, 2045, True, (256, 192)),
+    (8244, 2045, True, (256, 128)),      # the last tile 52 columns
+    (8192, 2048, False, (256, 256)),
+    (8192, 2045, True, (256, 256)),
+    (8180, 2045, True, (256, 256)),      # the last tile 244 columns
+    (5120, 2048, True, (256, 256)),
 ])
-def test_tiles_that_end_in_quads_equal_those_that_do_not(ctx, d, T, residual):
+def test_tiles_that_end_in_quads_equal_those_that_do_not(ctx, d, T, residual, tile):
     """The many-row kernel ends a whole tile on 16-byte boundaries with all its reads in front, any other element by
     element: the same call at an odd column of an odd row length gives the same bits, and rows past the active ones
     keep theirs."""
@@ -442,7 +446,28 @@ def test_tiles_that_end_in_quads_equal_those_that_do_not(ctx, d, T, residual):
     proj._gemm([w], x, a, T, d, 0, epilogue)
     proj._gemm([w], x, b, T, d + 3, 1, epilogue)
     ctx.sync()
+    assert last_tile(ctx) == tile
     a, b = a.get().reshape(batch, d), b.get().reshape(batch, d + 3)
     assert np.array_equal(a.view(np.uint32), np.ascontiguousarray(b[:, 1:d + 1]).view(np.uint32))
     assert np.array_equal(a[T:], start[T:]) and not np.array_equal(a[T - 1], start[T - 1])
     assert (b[:, 0] == UNTOUCHED).all() and (b[:, d + 1:] == UNTOUCHED).all()
+
+
+def test_the_largest_tile_adds_scaled_rows_to_what_is_there(ctx):
+    """256 x 256 tiles over fp32 activations whose rows have scales of their own, added to C: whole tiles and a last one of
+    244 columns and 253 rows."""
+    from jitllm_amd import synthetic
+    from jitllm_amd.projections import QuantizedBatchProjections
+    d, n, T = 8180, 256, 2045
+    say("largest tile, residual, fp32", d, n, T)
+    raw = synthetic.weight(O.Q8_0, d, n, seed=1795)
+    w = ctx.load_weight(O.Q8_0, raw, d, n)
+    X = synthetic.activations((T, n), seed=1796) * np.exp2(np.arange(T) % 11 - 5).astype(np.float32)[:, None]
+    start = synthetic.activations((T, d), seed=1797)
+    out = ctx.from_numpy(start)
+    proj = QuantizedBatchProjections(ctx, T, n, d)
+    proj.projection(ctx.from_numpy(X), out, w, n, d, True, T)
+    ctx.sync()
+    assert last_tile(ctx) == (256, 256)
+    got = out.get().reshape(T, d).astype(np.float64) - start
+    assert rel_err(got, O.matmul_batch(O.Q8_0, raw, X, d, n), magnitude(O.Q8_0, raw, X, d, n)) < F16_BOUND
