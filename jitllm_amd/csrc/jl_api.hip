@@ -114,6 +114,7 @@ int jl_context_set_split_k(jl_context *ctx, int enabled) {
 
 int jl_context_last_gemm(const jl_context *ctx) { return ctx ? ctx->last_gemm.load(std::memory_order_relaxed) : 0; }
 int jl_context_last_tile(const jl_context *ctx) { return ctx ? ctx->last_tile.load(std::memory_order_relaxed) : 0; }
+int jl_context_last_grid(const jl_context *ctx) { return ctx ? ctx->last_grid.load(std::memory_order_relaxed) : 0; }
 
 int jl_device_info(jl_context *ctx, int *compute_units, char *name, size_t name_bytes) {
     JL_REQUIRE(ctx != nullptr, "jl_device_info: context is null");

@@ -1409,6 +1409,7 @@ int launch_tiles_of(jl_context *ctx, const GemvParams &p, int threads, int lds, 
     int total = p.seg_tile_begin[p.nseg];
     int grid = ctx->compute_units * per_cu;
     if (grid > total) grid = total;
+    ctx->last_grid.store(grid, std::memory_order_relaxed);
     if (cells) {
         if (grid > *cells) return JL_NO_CELLS_FORM;   // more workgroups than the caller has cells for
         *cells = grid;

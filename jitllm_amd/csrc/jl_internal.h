@@ -32,6 +32,8 @@ struct jl_context {
     std::atomic<int> last_gemm{0};
     // rows * 1000 + columns of the tile of the last call that jl_gemm_hh took, for the tests (jl_context_last_tile)
     std::atomic<int> last_tile{0};
+    // workgroups of the last launch of jl_gemv_tiles, for the tests (jl_context_last_grid)
+    std::atomic<int> last_grid{0};
 };
 #define JL_GEMM_STREAMED 1          // jl_gemm_skinny
 #define JL_GEMM_IN_LOOP 2           // jl_gemm_f16
@@ -39,6 +41,7 @@ struct jl_context {
 #define JL_GEMM_IN_REGISTERS 100    // jl_gemm_reg: this and the number of its tiling
 extern "C" int jl_context_last_gemm(const jl_context *ctx);
 extern "C" int jl_context_last_tile(const jl_context *ctx);
+extern "C" int jl_context_last_grid(const jl_context *ctx);
 #define JL_CONTEXT_SCRATCH_BYTES 8192
 #define JL_CONTEXT_ARRIVALS 1024
 #define JL_BOUNCE_HALF_BYTES (8u << 20)

@@ -27,6 +27,11 @@ def last_tile(ctx) -> tuple:
     return divmod(ctx._lib.jl_context_last_tile(ctx.handle), 1000)
 
 
+def last_grid(ctx) -> int:
+    """Workgroups of the last single-token launch of the tile kernel."""
+    return ctx._lib.jl_context_last_grid(ctx.handle)
+
+
 def magnitude(t: int, raw: np.ndarray, X: np.ndarray, d: int, n: int) -> np.ndarray:
     """sum_j |w_ij x_bj| in float64, [B x d] (or [d] for a vector)."""
     w = np.abs(NP.DEQUANT[t](raw).reshape(d, n).astype(np.float64))

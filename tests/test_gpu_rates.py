@@ -1,11 +1,11 @@
-"""What a call takes against another call of the same kernel.
+"""What no comparison of results shows: what a call takes against another call of the same kernel, and how wide a grid is.
 
-Times of one box compared with each other, the least of several replays each: a call whose neighbour in size takes
-a fifth less per column has lost something that no comparison of results shows."""
+Times of one box are compared with each other, the least of several replays each: a call whose neighbour in size takes
+a fifth less per column has lost something."""
 import numpy as np
 import pytest
 
-from gpu_util import DECODED, last_gemm, say
+from gpu_util import DECODED, last_gemm, last_grid, say
 from oracle import pyoracle as O
 
 pytestmark = pytest.mark.gpu
@@ -66,3 +66,29 @@ def test_rows_no_power_of_two_apart_cost_no_more_per_column(ctx, hip, hidden, ro
         for w in sum(pairs, []):
             w.free()
     assert per_column[2560] < 1.14 * per_column[2048], per_column
+
+
+@pytest.mark.parametrize("t,d,n,two,workgroups", [
+    (O.Q8_0, 8192, 2048, True, 3),       # (four fit since its tiles come in by buffer loads; three are faster)
+    (O.Q4_0, 8960, 768, True, 3),
+    (O.Q6_K, 8192, 2048, True, 3),
+    (O.Q8_0, 16384, 2048, False, 4),     # what the LDS holds
+    (O.Q4_K, 32768, 768, False, 5),      # what 96 registers a lane allow
+    (O.Q4_K, 24576, 1536, False, 5),
+])
+def test_workgroups_a_compute_unit(ctx, t, d, n, two, workgroups):
+    """Launches of more tiles than the chip holds workgroups: gate/up takes three a compute unit, others as many as fit."""
+    from jitllm_amd import _lib as L, synthetic
+    say("workgroups", t, d, n, two)
+    raw = synthetic.weight(t, d, n, seed=2110)
+    w = [ctx.load_weight(t, raw, d, n) for _ in range(2 if two else 1)]
+    x, out = ctx.from_numpy(synthetic.activations(n, seed=2111)), ctx.float_array(d)
+    if two:
+        L.check(ctx._lib.jl_gemv_gate_up(ctx.handle, w[0].handle, w[1].handle, x.ptr, out.ptr))
+    else:
+        L.check(ctx._lib.jl_gemv(ctx.handle, w[0].handle, x.ptr, out.ptr, L.JL_STORE))
+    ctx.sync()
+    units, _ = ctx.device_info()
+    assert last_grid(ctx) == workgroups * units
+    for weight in w:
+        weight.free()
